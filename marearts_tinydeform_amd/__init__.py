@@ -30,7 +30,7 @@ MODES = ('auto', 'fused', 'project')
 # and checked on a grid of shapes the fit never saw (bench.py --holdout).
 FUSED_LIMIT = {
     torch.float32: {'fused': (3.7445, 7.6027, 0.0, 7.5341, 8.5712, 0.0, 0.4613, 0.0809, 3.7466),
-                    'gemm': (3.358, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 9.0783, 0.0612, 0.6669, 8.083),
+                    'gemm': (3.358, 0.34, 0.0, 0.0, 0.0, 0.0, 0.0, 9.0783, 0.0612, 0.6669, 8.083),
                     'sample': (2.6256, 0.0528, 0.0, 0.0134, 0.1157),
                     'gap': (0.408, 0.0131, 0.1278, 0.0015)},
     torch.float16: {'fused': (3.5241, 8.2634, 0.0, 7.7144, 8.1228, 0.0, 0.4747, 0.1105, 1.7771),
@@ -91,7 +91,7 @@ def cost_features(B, Q, H, D, C, N, L, P, s, aligned=True):
         proj_mflop the busiest CU's projection work, its workgroups' rows (at least one 16-row MFMA tile each) x C x D
       gemm   [1, stream_mb, tiled_busy_gflop, tiled_mb, deep_rounds, deep_rounds_k, deep_mb, f32_busy_gflop, f32_mb,
               other_gflop, f32_direct_busy_gflop]
-        terms of the kernel the value-projection size rule picks: the streaming kernel's bytes in whole 32-token steps
+        terms of the kernel the value-projection size rule picks: the streaming kernels' bytes in whole 32-token steps
         per CU; the tiled 16-bit kernels' flops in the busiest CU's tile count (times the CU count) and their bytes;
         the deep-K direct-to-LDS kernels' tile rounds on the busiest CU, those times K / 1e3, and their bytes;
         float32 tiles (busiest CU and bytes, as for 16 bits; the 64 x 128 tiles that read A straight from memory in a
@@ -117,7 +117,8 @@ def cost_features(B, Q, H, D, C, N, L, P, s, aligned=True):
     v = _native.value_proj_plan(pdt, M, K, NO, heads=H if hm else None, N=N if hm else None) if M * NO > 0 else -1
     mb, gf = M * (K + NO) * s / 1e6, 2.0 * M * K * NO / 1e9
     gemm = [1.0] + [0.0] * 10
-    if v == 22:
+    split = s == 4 and v > 0 and NO == 256 and K in (128, 256) and M >= 4500 and not hm  # float32 on split operands
+    if v == 22 or split:
         gemm[1] = -(-(-(-M // CUS)) // 32) * 32 * (K + NO) * s * CUS / 1e6
     elif v in (14, 18):
         mt, nt = -(-M // 256), -(-NO // 256)

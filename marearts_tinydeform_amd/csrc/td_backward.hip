@@ -2132,18 +2132,27 @@ int launch_transpose(int dtype, const void* src, void* dst, int64_t R, int64_t C
 
 // grad_memory = G . W (through W^T, as td_input_grad computes it) and the weight gradient of the same G: where the
 // value projection's size rule picks the 64 x 64 two-stage tiles for the input gradient, its tiles and the weight
-// gradient's run in one launch (input_weight_grad_kernel); otherwise the two run one after the other. The workspace
+// gradient's run in one launch (input_weight_grad_kernel), except in float32 where the split kernel is the faster one
+// for the input gradient; otherwise the two run one after the other. The workspace
 // is the weight gradient's (td_weight_grad_workspace). M, HD and C are positive.
 int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, const void* X, void* gm, void* gw,
                              void* gb, int64_t M, int64_t HD, int64_t C, void* workspace, int64_t ws_bytes,
                              hipStream_t stream) {
+    // grad_memory = G . W with W read as stored
+    const GemmParams sp{G, W, nullptr, gm, static_cast<int>(M), static_cast<int>(HD), static_cast<int>(C), 0, 0, 0};
+    int rc = 0;
+    if (dtype == kF32 && gemm_split_pays(sp)) {
+        rc = launch_gemm_split(sp, stream, true);
+        if (rc != 0) return rc;
+        return launch_wgrad(dtype, G, X, gw, gb, M, HD, C, workspace, ws_bytes, stream);
+    }
     if (value_proj_plan(dtype, G, Wt, nullptr, gm, M, HD, C, 0, 0) == 25) {
         // 16-bit with C a multiple of 8 and W 16-byte aligned: the GEMM reads W as stored (no transpose launch,
         // Wt is left unwritten)
         const bool stored = (dtype == kF16 || dtype == kBF16) && C % 8 == 0 &&
                             reinterpret_cast<uintptr_t>(W) % 16 == 0;
         if (!stored) {
-            const int rc = launch_transpose(dtype, W, Wt, HD, C, stream);
+            rc = launch_transpose(dtype, W, Wt, HD, C, stream);
             if (rc != 0) return rc;
         }
         const GemmParams gp{G, stored ? W : Wt, nullptr, gm, static_cast<int>(M), static_cast<int>(HD),
@@ -2151,8 +2160,6 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
         return launch_wgrad(dtype, G, X, gw, gb, M, HD, C, workspace, ws_bytes, stream, &gp, stored);
     }
     // the streaming GEMM (16-bit, C = 256, HD = 128 or 256, many tokens) reads W as stored too
-    const GemmParams sp{G, W, nullptr, gm, static_cast<int>(M), static_cast<int>(HD), static_cast<int>(C), 0, 0, 0};
-    int rc = 0;
     if (value_proj_plan(dtype, G, W, nullptr, gm, M, HD, C, 0, 0) == 22 && gemm_stream_fits(dtype, sp)) {
         rc = launch_gemm_stream(dtype, sp, stream, true);
         if (rc != 0) return rc;

@@ -89,4 +89,10 @@ bool gemm_stream_fits(int dtype, const GemmParams& p);
 // w_stored: p.w is [K, 256] as its owner stores it (C = A . W) instead of [256, K]
 int launch_gemm_stream(int dtype, GemmParams p, hipStream_t stream, bool w_stored = false);
 
+// Its float32 counterpart on split operands (td_gemm_split.hip): NO = 256, K = 128 or 256, row-major output, 16-byte
+// aligned a, w and c (gemm_split_fits); gemm_split_pays also asks for the rows from which it is the faster kernel.
+bool gemm_split_fits(const GemmParams& p);
+bool gemm_split_pays(const GemmParams& p);
+int launch_gemm_split(GemmParams p, hipStream_t stream, bool w_stored = false);
+
 }  // namespace td

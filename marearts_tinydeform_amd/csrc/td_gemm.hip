@@ -254,12 +254,12 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //       against 14.2), then both operands through LDS with K chunks of 128 (9) while under 512 tiles of 128 x 128
 //       (M = 3600: 19.4 against 25.9; against the direct-to-LDS kernel, K = NO = 512: M = 2400 8.1 against 13.1,
 //       M = 4800 11.5 against 13.6; K = NO = 1024: M = 1800 12.8 against 20.0, M = 3600 18.9 against 21.9), else 13.
-// float32 (MFMA-bound: v_mfma_f32_16x16x4_f32), by the count of 64 x 64 tiles: K <= 256: up to 40 tiles 32 x 32 (24)
+// float32 (bound by v_mfma_f32_16x16x4_f32), by the count of 64 x 64 tiles: K <= 256: up to 40 tiles 32 x 32 (24)
 //   (K = NO = 256: M = 300 6.0 µs against 9.4 for 5), up to 100 64 x 32 (23) (M = 1200 6.8 against 9.5), up to 1100
-//   two-stage 64 x 64 (25) (M = 2400 9.2 against 9.7, M = 8400 19.8 against 20.9), then 64 x 64 one-chunk tiles (5)
-//   under 1024 tiles of 128 x 128 (M = 33600 54.4 against 56.2), else A direct in 64 x 128 tiles (2) (M = 67200: 93.5
-//   against 96.4); K >= 512: two-stage 64 x 64 (25) under 512 tiles (M = 600, K = NO = 1024: 27.2 against 48.8 for
-//   2), else 2.
+//   two-stage 64 x 64 (25) (M = 2400 9.2 against 9.7), then 64 x 64 one-chunk tiles (5) under 1024 tiles of 128 x 128
+//   (M = 33600 54.4 against 56.2), else A direct in 64 x 128 tiles (2); K >= 512: two-stage 64 x 64 (25) under 512
+//   tiles (M = 600, K = NO = 1024: 27.2 against 48.8 for 2), else 2. Of these, products that the split kernels compute
+//   faster on the bfloat16 units (gemm_split_pays) run there instead.
 int pick_variant(int dtype, const GemmParams& p) {
     if (dtype != kF32 && dtype != kF16 && dtype != kBF16) return 0;
     const int E = dtype == kF32 ? 4 : 8;
@@ -284,6 +284,9 @@ template <typename T>
 int launch_t(GemmParams p, hipStream_t stream, int variant) {
     constexpr int dt = std::is_same<T, float>::value ? kF32 : std::is_same<T, f16>::value ? kF16
                        : std::is_same<T, bf16>::value ? kBF16 : kF64;
+    if constexpr (dt == kF32) {
+        if (variant != 0 && gemm_split_pays(p)) return launch_gemm_split(p, stream);
+    }
     if constexpr (!std::is_same<T, double>::value) {
         switch (variant) {
             case 0: break;
