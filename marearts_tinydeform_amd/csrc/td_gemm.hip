@@ -29,7 +29,7 @@ __global__ __launch_bounds__(WM* WN* kWave) void gemm_lds_kernel(GemmParams p) {
     constexpr int KBK = KBlock<T>::kK;
     constexpr int KC = NKB * KBK;
     constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    constexpr int LDK = KC + E;
+    constexpr int LDK = KC + 2 * E;  // 32 bytes of padding: full-rate fragment reads (as in GemmMfmaTile)
     constexpr int A_CHUNKS = BM * KC / E, B_CHUNKS = BN * KC / E;
     constexpr int A_PER_T = (A_CHUNKS + NTH - 1) / NTH, B_PER_T = (B_CHUNKS + NTH - 1) / NTH;
     constexpr int LDC = BN + E;

@@ -14,6 +14,8 @@ namespace td {
 //   W  the workgroup stages the BN x chunk slice in LDS (two buffers, filled from registers one chunk ahead).
 // STAGES = 2 overlaps the next chunk's loads with this chunk's MFMAs; STAGES = 1 (one LDS buffer) suits K that fits
 // one chunk, where the whole product costs a single round trip to memory.
+// A staged W row is 32 bytes longer than its chunk: the 16 rows of a fragment read then go at the full LDS rate, where
+// with 16 bytes they took twice as long (525 against 290 B/ns a CU in a probe of the reads alone).
 // Epilogue: bias, one rounding to T, the tile transposed through LDS and written with 16-byte stores.
 // DUAL: C = A . W^T + A2 . W^T + bias with A2 the same shape as A (two MFMAs per block; the sum A + A2 is never
 // rounded to T). F32OUT: C is float32, the accumulators stored unrounded.
@@ -33,7 +35,7 @@ struct GemmMfmaTile {
     static constexpr int KBK = KBlock<T>::kK;                   // K per 16-byte block (4 lane groups)
     static constexpr int KC = NKB * KBK;                         // K per chunk
     static constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
-    static constexpr int LDK = KC + E;                           // LDS pitch (elements) of a staged W row
+    static constexpr int LDK = KC + 2 * E;                          // LDS pitch (elements) of a staged W row
     static constexpr int LDN = BN + 16;                          // WT: LDS pitch (elements) of a staged k row
     static constexpr int B_CHUNKS = BN * KC / E;                 // 16-byte pieces of one staged W slice
     static constexpr int B_PER_T = (B_CHUNKS + NTH - 1) / NTH;
