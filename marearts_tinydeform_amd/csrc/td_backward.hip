@@ -704,7 +704,6 @@ __global__ __launch_bounds__(256) void loc_attn_backward_kernel(LocAttnParams lp
 // D is a power of two from 4 to 64 (lane = channel tid % D), P > 0. The sums reach grad_value in another order than
 // the direct scatter's, so the two agree to float rounding.
 constexpr int kBucketPix = 1024;  // bounding-box pixels per level at most
-constexpr int kTileW = 8, kTileH = 4;  // self-attention tiles: 8 x 4 pixels of a level's map (QT = 32 queries)
 constexpr int kBucketEnt = 1024;  // corner entries per level at most: QT * P * 4 with QT * L * P <= 256
 
 // a bucketed corner: its coefficient a * w_c and the offset of its grad_out row in LDS (r * D)
@@ -759,7 +758,7 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
-template <typename T, int NTH, bool TILE2D>
+template <typename T, int NTH>
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void scatter_bucket_kernel(BucketParams bp) {
     using A = float;
     constexpr int NW = NTH / kWave;
@@ -968,44 +967,381 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void s
         }
     };
 
-    if constexpr (!TILE2D) {
-        // QT consecutive queries
-        const int unit = (blockIdx.x % kXcds) * bp.per_xcd + blockIdx.x / kXcds;
-        if (unit >= bp.units) return;  // the whole workgroup
-        const int qt = unit % bp.qtiles, bh = unit / bp.qtiles;
-        const int q0 = qt * QT, nq = g.Q - q0 < QT ? g.Q - q0 : QT;
-        tile(bh / g.H, bh % g.H, [&](int r) { return r < nq ? q0 + r : -1; });
-    } else {
-        // self-attention (Q = N, query q at token q's pixel): tiles of kTileW x kTileH pixels of each level's map, in
-        // level order; the level sizes are on the device, so every workgroup counts the tiles and takes every
-        // gridDim.x-th
-        auto level_tiles = [&](int l, int& nbx) {
-            const int wl = static_cast<int>(g.shapes[2 * l + 1]), hl = static_cast<int>(g.shapes[2 * l]);
-            nbx = (wl + kTileW - 1) / kTileW;
-            return nbx * ((hl + kTileH - 1) / kTileH);
-        };
-        int per_bh = 0;
-        for (int l = 0; l < g.L; ++l) {
-            int nbx;
-            per_bh += level_tiles(l, nbx);
+    const int unit = (blockIdx.x % kXcds) * bp.per_xcd + blockIdx.x / kXcds;
+    if (unit >= bp.units) return;  // the whole workgroup
+    const int qt = unit % bp.qtiles, bh = unit / bp.qtiles;
+    const int q0 = qt * QT, nq = g.Q - q0 < QT ? g.Q - q0 : QT;
+    tile(bh / g.H, bh % g.H, [&](int r) { return r < nq ? q0 + r : -1; });
+}
+
+// The same scatter for self-attention (Q = N, query q at token q's pixel), a workgroup a tile of 16 x 16 or 16 x 8
+// pixels of a level's map: those queries of one head touch 10.2 and 7.9 times fewer pixels than they have corners on
+// DINO-style inputs (8 x 4 pixels: 4.3), and the float atomics, one D-wide line a touched pixel, run at 320 G lanes/s
+// whatever else is done (200 and 260 us at the DINO encoder). So the rest has to run beside them: the barriers wait for
+// LDS only, nothing inside a tile waits for a load, and a level costs three barriers:
+//   * a thread a sample: its corners inside the level's window rank themselves within their pixel (an integer LDS
+//     atomic each); a corner outside it is listed for an atomic of its own. The window is the tile's image on the
+//     level and a margin, up to kPix pixels: known beforehand, and a stray corner costs one line, where a bounding box
+//     that it stretched would cost the level;
+//   * a thread 4 pixels: each wavefront scans its counts and takes that much of the entry and pixel lists by one
+//     atomic, so no scan over the workgroup;
+//   * the entries go to their pixel's place;
+//   * D / 8 lanes a touched pixel sum its entries, 8 channels a lane, the pixels in order of their counts so that a
+//     wavefront's lanes take about as many rounds, and those with 8 and 16 entries or more in two and four streams;
+//     the sums are turned by LDS so that an atomic instruction adds whole lines.
+// Levels that a window cannot cover (coarse queries on fine levels, a few percent of them) add mostly directly.
+// At the DINO encoder (2 x 22223 queries, fp16): 561 us with scatter_bucket_kernel in 8 x 4-pixel tiles -> 276 (16 x 16;
+// 299 with 16 x 8), training step 837 -> 543. Copies without the atomics take 232 (16 x 8), without the sums and them
+// 135: no one part bounds it. Entries summed pixel by pixel without the order and the streams: 350.
+// For NTH threads: pixels of a window, corners of a level (4 a thread) and grad_out channels of a tile at most
+template <int NTH>
+struct TileShape {
+    static constexpr int kPix = 4 * NTH, kEnt = 4 * NTH, kGrad = 8 * NTH;
+    static constexpr int kSide = NTH >= 1024 ? 64 : 45;  // kSide * kSide <= kPix
+};
+constexpr int kTileMargin = 16;
+constexpr int kAhead = 4;                   // levels whose samples are loaded together
+
+struct TileParams {
+    const void* loc;
+    const void* attn;
+    const void* grad_out;
+    void* grad_value;  // [B, N, H * D] float, zeroed
+    Geom g;
+    int tw, th, tw_shift, th_shift, d_shift;  // tile: tw * th * P <= NTH, tw * th * D <= kGrad; logs of 2
+    FastDiv d_p;
+};
+
+// This wavefront's LDS accesses done, then a barrier that leaves its loads and atomics in flight
+__device__ __forceinline__ void meet_lds() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Touched pixels are listed by their number of entries, so that the pixels a wavefront sums together take about as
+// many rounds: class c, from 2^c entries on, in a part of the list that holds as many as there can be
+constexpr int kTileClasses = 6;
+template <typename T, int NTH>
+struct TileLds : TileShape<NTH> {
+    using S = TileShape<NTH>;
+    __host__ __device__ static constexpr int class_at(int c) { return 2 * S::kEnt - (2 * S::kEnt >> c); }
+    static constexpr int kList = 2 * S::kEnt - (2 * S::kEnt >> kTileClasses);
+    alignas(16) T gr[S::kGrad];                // [QT][D]
+    int cnt[S::kPix];                          // corners per window pixel; zero between levels
+    union {
+        int base[S::kPix];                     // start of the pixel's entries
+        float turned[S::kPix];                 // then sums by lines: 4 * kWave a wavefront
+    };
+    BucketEntry lent[S::kEnt];                 // entries by pixel; direct corners from the end
+    int tinfo[kList];                          // touched pixels: start | count << 16; class 0's last: the direct
+                                               // corners' rows
+    int tat[kList];                            // touched pixels: row, as an element offset in the image's gradient
+    int alloc[2], ndirect[2];                  // by turns of the levels: entries placed; direct corners
+    int touched[2][8];                         // and pixels listed by class
+};
+
+template <typename T, int NTH>
+__global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
+    using A = float;
+    using Lds = TileLds<T, NTH>;
+    constexpr int kTileThreads = NTH, kTilePix = Lds::kPix, kTileEnt = Lds::kEnt, kSide = Lds::kSide;
+    const Geom& g = tp.g;
+    const int D = g.D, HD = g.H * g.D, P = g.P, QT = tp.tw * tp.th;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & (kWave - 1);
+
+    extern __shared__ __align__(16) unsigned char smem[];
+    Lds& s = *reinterpret_cast<Lds*>(smem);
+
+    const T* __restrict__ go = static_cast<const T*>(tp.grad_out);
+    for (int i = tid; i < kTilePix; i += kTileThreads) s.cnt[i] = 0;
+    if (tid < 2) s.alloc[tid] = s.ndirect[tid] = 0;
+    if (tid < 16) s.touched[0][tid] = 0;
+
+    // lane l's: level l's size and first token, read once (a load would wait for the atomics before it); L <= 64
+    const int ll = lane < g.L ? lane : 0;
+    const int level_w = static_cast<int>(g.shapes[2 * ll + 1]), level_h = static_cast<int>(g.shapes[2 * ll]);
+    const int64_t level_st = g.starts[ll];
+    const int level_lo = static_cast<int>(level_st), level_hi = static_cast<int>(level_st >> 32);
+    auto width = [&](int l) { return __builtin_amdgcn_readlane(level_w, l); };
+    auto height = [&](int l) { return __builtin_amdgcn_readlane(level_h, l); };
+    auto start = [&](int l) {
+        return static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(level_lo, l))) |
+               static_cast<int64_t>(__builtin_amdgcn_readlane(level_hi, l)) << 32;
+    };
+    auto level_tiles = [&](int l, int& nbx) {
+        nbx = (width(l) + tp.tw - 1) >> tp.tw_shift;
+        return nbx * ((height(l) + tp.th - 1) >> tp.th_shift);
+    };
+    int per_bh = 0;
+    for (int l = 0; l < g.L; ++l) {
+        int nbx;
+        per_bh += level_tiles(l, nbx);
+    }
+    const int tiles = g.B * g.H * per_bh;
+    int par = 0;
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int bh = t / per_bh, b = bh / g.H, h = bh - b * g.H;
+        int rest = t - bh * per_bh, lq = 0, nbx = 1;
+        for (; lq < g.L; ++lq) {
+            const int n = level_tiles(lq, nbx);
+            if (rest < n) break;
+            rest -= n;
         }
-        const int tiles = g.B * g.H * per_bh;
-        for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-            __syncthreads();  // every wavefront is done with the previous tile's LDS
-            const int bh = t / per_bh;
-            int rest = t - bh * per_bh, lq = 0, nbx = 1;
-            for (; lq < g.L; ++lq) {
-                const int n = level_tiles(lq, nbx);
-                if (rest < n) break;
-                rest -= n;
+        const int wq = width(lq), hq = height(lq);
+        const int qx = (rest % nbx) * tp.tw, qy = (rest / nbx) * tp.th;
+        const int nx = min(tp.tw, wq - qx), ny = min(tp.th, hq - qy);
+        const int64_t stq = start(lq);
+        // the query of row r; -1: none (past the map, or a token that is not in [0, N))
+        auto query_of = [&](int r) {
+            const int y = r >> tp.tw_shift, x = r & (tp.tw - 1);
+            const int64_t q = stq + static_cast<int64_t>(qy + y) * wq + qx + x;
+            return x < nx && y < ny && q >= 0 && q < g.Q ? static_cast<int>(q) : -1;
+        };
+        A* __restrict__ gv =
+            static_cast<A*>(tp.grad_value) + static_cast<int64_t>(b) * g.N * HD + static_cast<int64_t>(h) * D;
+
+        // lane l's: the window on level l, the tile's pixel centres there and a margin, inside the map
+        int wx0, wy0, wbw, wbh;
+        {
+            const int wl = level_w, hl = level_h;
+            const A sx = static_cast<A>(wl) / static_cast<A>(wq), sy = static_cast<A>(hl) / static_cast<A>(hq);
+            int xa = static_cast<int>(floorf((qx + 0.5f) * sx - 0.5f));
+            int xb = static_cast<int>(floorf((qx + nx - 0.5f) * sx - 0.5f)) + 1;
+            int ya = static_cast<int>(floorf((qy + 0.5f) * sy - 0.5f));
+            int yb = static_cast<int>(floorf((qy + ny - 0.5f) * sy - 0.5f)) + 1;
+            const int cx = (xa + xb) / 2, cy = (ya + yb) / 2;
+            if (xb - xa + 1 > kSide) xa = cx - (kSide - 1) / 2, xb = cx + (kSide - 1) / 2;  // around the centre
+            if (yb - ya + 1 > kSide) ya = cy - (kSide - 1) / 2, yb = cy + (kSide - 1) / 2;
+            // the widest margin m with (w + 2 m)(h + 2 m) <= kTilePix
+            const A w = static_cast<A>(xb - xa + 1), d = static_cast<A>(yb - ya + 1);
+            int m = static_cast<int>((sqrtf((w - d) * (w - d) + 4.f * kTilePix) - (w + d)) * 0.25f);
+            m = min(max(m, 0), kTileMargin);
+            wx0 = max(xa - m, 0), wy0 = max(ya - m, 0);
+            wbw = max(min(xb + m, wl - 1) - wx0 + 1, 0), wbh = max(min(yb + m, hl - 1) - wy0 + 1, 0);
+            if (wbw * wbh > kTilePix) wbw = wbh = 0;  // rounding only: every corner then goes directly
+        }
+
+        // this thread's samples: point jp of row r, level by level
+        const int r = static_cast<int>(fast_div(tp.d_p, static_cast<uint32_t>(tid))), jp = tid - r * P;
+        const int q = r < QT ? query_of(r) : -1;
+        const int64_t first = ((static_cast<int64_t>(b) * g.Q + (q >= 0 ? q : 0)) * g.H + h) * g.LP + jp;
+        // the samples of kAhead levels, loaded and waited for before any of their atomics: a wavefront's vector memory
+        // operations complete in order, and a wait inside the levels' loop would be one for the atomics
+        using Bits = typename std::conditional<sizeof(T) == 2, uint16_t, uint32_t>::type;
+        const Bits* const lbits = static_cast<const Bits*>(tp.loc);
+        const Bits* const abits = static_cast<const Bits*>(tp.attn);
+        uint32_t rx[kAhead], ry[kAhead], ra[kAhead];
+        auto load = [&](int l0) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const bool on = q >= 0 && l0 + u < g.L;
+                const int64_t i = first + (on ? l0 + u : 0) * P;
+                rx[u] = on ? lbits[2 * i] : 0u;
+                ry[u] = on ? lbits[2 * i + 1] : 0u;
+                ra[u] = on ? abits[i] : 0u;
             }
-            const int wl = static_cast<int>(g.shapes[2 * lq + 1]), hl = static_cast<int>(g.shapes[2 * lq]);
-            const int x0 = (rest % nbx) * kTileW, y0 = (rest / nbx) * kTileH;
-            const int st = static_cast<int>(g.starts[lq]);
-            tile(bh / g.H, bh % g.H, [&](int r) {
-                const int x = x0 + r % kTileW, y = y0 + r / kTileW;
-                return x < wl && y < hl ? st + y * wl + x : -1;
-            });
+        };
+        auto loaded = [&] {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) asm volatile("" : "+v"(rx[u]), "+v"(ry[u]), "+v"(ra[u]));
+        };
+        load(0);
+        meet_lds();  // every wavefront is done with the previous tile's rows
+        for (int i = tid; i < QT * D; i += kTileThreads) {
+            const int row = i >> tp.d_shift, qr = query_of(row);
+            s.gr[i] = qr >= 0 ? go[(static_cast<int64_t>(b) * g.Q + qr) * HD + static_cast<int64_t>(h) * D + (i - row * D)]
+                              : T(0);
+        }
+
+        loaded();
+        for (int l = 0; l < g.L; ++l, par ^= 1) {
+            const int wl = width(l), hl = height(l);
+            const int64_t st = start(l);
+            if (l > 0 && l % kAhead == 0) {
+                load(l);
+                loaded();
+            }
+            const int x0 = __builtin_amdgcn_readlane(wx0, l), y0 = __builtin_amdgcn_readlane(wy0, l);
+            const int bw = __builtin_amdgcn_readlane(wbw, l), bh_ = __builtin_amdgcn_readlane(wbh, l);
+            // corner k: px its window pixel (-1: none, or outside the window), rank its place among the pixel's
+            // entries or, outside the window, in the direct list; tk a direct corner's token
+            int tk[4] = {-1, -1, -1, -1}, px[4] = {-1, -1, -1, -1}, rank[4];
+            // a padding mask, or a level that is not all of it in [0, N): each corner's token is looked at
+            const bool checked = g.mask != nullptr || st < 0 || st + static_cast<int64_t>(wl) * hl > g.N;
+            A cf[4];
+            if (q >= 0) {
+                uint32_t tx = rx[0], ty = ry[0], ta = ra[0];
+#pragma unroll
+                for (int u = 1; u < kAhead; ++u)
+                    if (l % kAhead == u) tx = rx[u], ty = ry[u], ta = ra[u];
+                auto value = [](uint32_t v) { return cvt<A>(__builtin_bit_cast(T, static_cast<Bits>(v))); };
+                const A lx = value(tx), ly = value(ty), la = value(ta);
+                const A x = fmin(fmax(lx * static_cast<A>(wl) - 0.5f, -2.f), static_cast<A>(wl) + 1.f);
+                const A y = fmin(fmax(ly * static_cast<A>(hl) - 0.5f, -2.f), static_cast<A>(hl) + 1.f);
+                const A xf = floor(x), yf = floor(y), fx = x - xf, fy = y - yf;
+                const int ix = static_cast<int>(xf), iy = static_cast<int>(yf);
+                const int wx = ix - x0, wy = iy - y0, at = wy * bw + wx;
+                bool all = true;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int dx = k & 1, dy = k >> 1;
+                    cf[k] = la * ((dx ? fx : 1.f - fx) * (dy ? fy : 1.f - fy));
+                    bool in = static_cast<unsigned>(wx + dx) < static_cast<unsigned>(bw) &&
+                              static_cast<unsigned>(wy + dy) < static_cast<unsigned>(bh_);
+                    all &= in;
+                    if (checked) {
+                        if (in) {
+                            const int64_t tok = st + static_cast<int64_t>(iy + dy) * wl + (ix + dx);
+                            in = tok >= 0 && tok < g.N &&
+                                 (g.mask == nullptr || g.mask[static_cast<int64_t>(b) * g.N + tok] == 0);
+                        }
+                    }
+                    if (in) {
+                        px[k] = at + dx + (dy ? bw : 0);
+                        rank[k] = atomicAdd(&s.cnt[px[k]], 1);
+                    }
+                }
+                if (!all) {  // corners outside the window, in the map or not
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int xi = ix + (k & 1), yi = iy + (k >> 1);
+                        const int64_t tok = st + static_cast<int64_t>(yi) * wl + xi;
+                        bool in = !(static_cast<unsigned>(xi - x0) < static_cast<unsigned>(bw) &&
+                                    static_cast<unsigned>(yi - y0) < static_cast<unsigned>(bh_)) &&
+                                  xi >= 0 && xi < wl && yi >= 0 && yi < hl;
+                        if (checked)
+                            in = in && tok >= 0 && tok < g.N &&
+                                 (g.mask == nullptr || g.mask[static_cast<int64_t>(b) * g.N + tok] == 0);
+                        if (in) {
+                            tk[k] = static_cast<int>(tok);
+                            rank[k] = atomicAdd(&s.ndirect[par], 1);
+                        }
+                    }
+                }
+            }
+            meet_lds();  // the counts (and, first, the grad_out rows) are in place; the last level's sums are done
+            {
+                const int4 c = reinterpret_cast<const int4*>(s.cnt)[tid];
+                const int own = c.x + c.y + c.z + c.w;
+                const int incl = wave_incl_scan(own);
+                int from = 0;
+                if (lane == kWave - 1 && incl != 0) from = atomicAdd(&s.alloc[par], incl);
+                int run = __builtin_amdgcn_readlane(from, kWave - 1) + incl - own;
+                if (own != 0) {
+                    const int cs[4] = {c.x, c.y, c.z, c.w};
+                    int bs[4];
+                    const int yy = static_cast<int>((4 * tid + 0.5f) * (1.f / static_cast<A>(bw)));  // 4 tid / bw
+                    int xx = 4 * tid - yy * bw;
+                    int tok = static_cast<int>(st) + (y0 + yy) * wl + x0 + xx;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        bs[i] = run;
+                        if (cs[i] > 0) {
+                            const int cl = min(31 - __builtin_clz(static_cast<unsigned>(cs[i])), kTileClasses - 1);
+                            const int at = Lds::class_at(cl) + atomicAdd(&s.touched[par][cl], 1);
+                            s.tinfo[at] = run | cs[i] << 16;
+                            s.tat[at] = tok * HD;
+                            run += cs[i];
+                        }
+                        ++tok;
+                        if (++xx == bw) xx = 0, tok += wl - bw;
+                    }
+                    reinterpret_cast<int4*>(s.base)[tid] = make_int4(bs[0], bs[1], bs[2], bs[3]);
+                    reinterpret_cast<int4*>(s.cnt)[tid] = make_int4(0, 0, 0, 0);
+                }
+                if (tid == 0) s.ndirect[par ^ 1] = 0;
+            }
+            meet_lds();  // every pixel has its place
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (px[k] >= 0) s.lent[s.base[px[k]] + rank[k]] = BucketEntry{cf[k], r * D};
+                if (tk[k] >= 0) {
+                    s.lent[kTileEnt - 1 - rank[k]] = BucketEntry{cf[k], r * D};
+                    s.tinfo[kTileEnt - 1 - rank[k]] = tk[k] * HD;
+                }
+            }
+            if (tid == 0) s.alloc[par ^ 1] = 0;
+            if (tid < 8) s.touched[par ^ 1][tid] = 0;
+            meet_lds();  // the entries are in place
+            // a wavefront's lanes in two halves, and a half in 256 / D rows of D / 8 lanes
+            const int lpr_shift = tp.d_shift - 3, rows = (4 * kWave) >> tp.d_shift;
+            const int row = (lane & 31) >> lpr_shift, sub = (lane & ((1 << lpr_shift) - 1)) * 8;
+            A* const turned = s.turned + wave * (4 * kWave);  // a half: [256 / D][D]
+            int turn = wave;  // the classes' groups of pixels go round the wavefronts, the longest first
+            // class cl, an entry list in S streams: row = stream * (rows / S) + pixel of the half
+            auto sum_class = [&](int cl, auto streams) {
+                constexpr int S = decltype(streams)::value;
+                const int total = s.touched[par][cl], ppw_shift = 9 - tp.d_shift - (S == 4 ? 2 : S == 2 ? 1 : 0);
+                const int groups = (total + (1 << ppw_shift) - 1) >> ppw_shift, pe = Lds::class_at(cl) + total;
+                const int half_px = rows / S, stream = row >> (ppw_shift - 1), px_row = row & (half_px - 1);
+                for (; turn < groups; turn += kTileThreads / kWave) {
+                    const int p0 = Lds::class_at(cl) + (turn << ppw_shift);
+                    const int pi = p0 + (lane >> 5) * half_px + px_row;
+                    f32x4 v[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+                    if (pi < pe) {
+                        const int info = s.tinfo[pi], n = info >> 16;
+                        const BucketEntry* const e = s.lent + (info & 0xffff);
+                        const T* const gs = s.gr + sub;
+                        auto add = [&](const BucketEntry& u) {  // 8 channels of the entry's row
+                            using T8 = T __attribute__((ext_vector_type(8)));
+                            const T8 g8 = *reinterpret_cast<const T8*>(gs + u.row);
+#pragma unroll
+                            for (int c = 0; c < 8; ++c) v[c >> 2][c & 3] = fmaf(u.coef, cvt<A>(g8[c]), v[c >> 2][c & 3]);
+                        };
+                        int i = stream;
+                        for (; i + 3 * S < n; i += 4 * S) {  // four entries' reads in flight
+                            const BucketEntry u0 = e[i], u1 = e[i + S], u2 = e[i + 2 * S], u3 = e[i + 3 * S];
+                            add(u0);
+                            add(u1);
+                            add(u2);
+                            add(u3);
+                        }
+                        if (i < n) {
+                            const BucketEntry u0 = e[i], u1 = e[min(i + S, n - 1)], u2 = e[min(i + 2 * S, n - 1)];
+                            add(u0);
+                            if (i + S < n) add(u1);
+                            if (i + 2 * S < n) add(u2);
+                        }
+                    }
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        if (lane >> 5 == half) {
+                            f32x4* const to = reinterpret_cast<f32x4*>(turned + 8 * (lane & 31));
+                            to[0] = v[0];
+                            to[1] = v[1];
+                        }
+                        asm volatile("" ::: "memory");  // the other lanes' stores: no load kept from before them
+                        A t[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) t[i] = turned[i * kWave + lane];
+                        asm volatile("" ::: "memory");
+#pragma unroll
+                        for (int i = 0; i < 4 / S; ++i) {  // the streams are rows of the same pixels
+                            A sum = t[i];
+                            if constexpr (S == 2) sum += t[i + 2];
+                            if constexpr (S == 4) sum = (t[0] + t[1]) + (t[2] + t[3]);
+                            const int pr = p0 + half * half_px + ((i * kWave + lane) >> tp.d_shift);
+                            if (pr < pe)
+                                atomic_add(gv + static_cast<unsigned>(s.tat[pr] + (lane & (D - 1))), sum);
+                        }
+                    }
+                }
+                turn -= groups;
+            };
+            sum_class(5, std::integral_constant<int, 4>{});
+            sum_class(4, std::integral_constant<int, 4>{});
+            sum_class(3, std::integral_constant<int, 2>{});
+            for (int cl = 2; cl >= 0; --cl) sum_class(cl, std::integral_constant<int, 1>{});
+            const int nd = s.ndirect[par];
+            for (int i = tid; i < nd * D; i += kTileThreads) {
+                const int at = kTileEnt - 1 - (i >> tp.d_shift), d = i & (D - 1);
+                const BucketEntry u = s.lent[at];
+                atomic_add(gv + static_cast<unsigned>(s.tinfo[at] + d), u.coef * cvt<A>(s.gr[u.row + d]));
+            }
         }
     }
 }
@@ -1861,9 +2197,50 @@ inline bool bucket_scatter_pays(const Geom& g) {
            static_cast<int64_t>(g.Q) * g.LP * 4 >= int64_t{16} * g.N;
 }
 
+// Self-attention (as many queries as tokens): scatter_tile_kernel, in the largest tile whose samples of a level have a
+// thread each and whose grad_out rows fit its LDS; 1 without launching when that is under 32 queries.
+template <typename T, int NTH>
+int scatter_tile_shape_go(const BackParams& p, hipStream_t stream) {
+    const Geom& g = p.g;
+    TileParams tp{p.loc, p.attn, p.grad_out, p.grad_value, g, 0, 0, 0, 0, ilog2(g.D),
+                  make_fastdiv(static_cast<uint32_t>(g.P))};
+    for (int qs = 8; qs >= 5 && tp.tw == 0; --qs)  // 16 x 16, 16 x 8, 8 x 8, 8 x 4
+        if ((g.P << qs) <= NTH && (g.D << qs) <= TileShape<NTH>::kGrad)
+            tp.tw_shift = (qs + 1) / 2, tp.th_shift = qs / 2, tp.tw = 1 << tp.tw_shift, tp.th = 1 << tp.th_shift;
+    if (tp.tw == 0) return 1;
+    static std::atomic<uint64_t> done{0};
+    const int lds = static_cast<int>(sizeof(TileLds<T, NTH>));
+    const hipError_t attr =
+        allow_dynamic_lds(reinterpret_cast<const void*>(scatter_tile_kernel<T, NTH>), lds, done);
+    if (attr != hipSuccess)
+        return set_error(-3, "sample backward: LDS size attribute refused: %s", hipGetErrorString(attr));
+    // about one workgroup a tile (a workgroup strides over the tiles: the levels' sizes, and with them the count,
+    // are on the device)
+    const int64_t grid = static_cast<int64_t>(g.B) * g.H * (((g.N - 1) >> (tp.tw_shift + tp.th_shift)) + 1 + 2 * g.L);
+    hipLaunchKernelGGL((scatter_tile_kernel<T, NTH>), dim3(static_cast<unsigned>(grid)), dim3(NTH), lds, stream, tp);
+    return launched("sample backward scatter");
+}
+
+template <typename T>
+int scatter_tile_go(const BackParams& p, hipStream_t stream) {
+    const Geom& g = p.g;
+    const int64_t rows = static_cast<int64_t>(g.B) * g.H * g.N;
+    if (g.Q != g.N || g.D < 8 || g.discrete || g.loc_acc || rows > (int64_t{1} << 30) ||
+        static_cast<int64_t>(g.N) * g.H * g.D > (int64_t{1} << 30))
+        return 1;
+    // 1024 threads (16 x 16-pixel tiles, one workgroup a CU; in float32 its LDS does not fit) where there are two
+    // tiles a CU: DINO encoder 276 us against 299 with 512 threads (16 x 8 pixels, two workgroups)
+    if constexpr (sizeof(T) == 2) {
+        if (rows >= 512 * static_cast<int64_t>(cu_count())) return scatter_tile_shape_go<T, 1024>(p, stream);
+    }
+    return scatter_tile_shape_go<T, 512>(p, stream);
+}
+
 template <typename T>
 int scatter_bucket_go(const BackParams& p, hipStream_t stream) {
     const Geom& g = p.g;
+    const int rc = scatter_tile_go<T>(p, stream);
+    if (rc != 1) return rc;
     BucketParams bp{p.loc, p.attn, p.grad_out, p.grad_value, g, 0, 0, 0, 0, {}, {}};
     constexpr int NTH = 512;
     // QT rows of one (row, sample) per thread, QT * P * 4 corner entries per level, QT * D grad_out floats
@@ -1880,19 +2257,7 @@ int scatter_bucket_go(const BackParams& p, hipStream_t stream) {
     bp.per_xcd = static_cast<int>((units + kXcds - 1) / kXcds);
     bp.d_lp = make_fastdiv(static_cast<uint32_t>(g.LP));
     bp.d_p = make_fastdiv(static_cast<uint32_t>(g.P));
-    // Self-attention (as many queries as tokens, 32-query tiles): 8 x 4-pixel tiles of each level's map, which touch
-    // fewer pixels than 32 queries along one map row and never wrap a row; the tile count depends on the level sizes,
-    // which stay on the device, so a grid of three workgroups per CU (what the kernel's registers allow) strides
-    // over them
-    if (g.Q == g.N && bp.QT == kTileW * kTileH && static_cast<int64_t>(g.B) * g.H * g.N <= (int64_t{1} << 30)) {
-        int64_t grid = static_cast<int64_t>(g.B) * g.H * ((g.N + bp.QT - 1) / bp.QT + 2 * g.L);
-        const int64_t resident = 3 * static_cast<int64_t>(cu_count());
-        if (grid > resident) grid = resident;
-        hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, true>), dim3(static_cast<unsigned>(grid)), dim3(NTH), 0,
-                           stream, bp);
-        return launched("sample backward scatter");
-    }
-    hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, false>), dim3(static_cast<unsigned>(bp.per_xcd * kXcds)),
+    hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH>), dim3(static_cast<unsigned>(bp.per_xcd * kXcds)),
                        dim3(NTH), 0, stream, bp);
     return launched("sample backward scatter");
 }

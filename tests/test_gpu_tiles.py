@@ -1,0 +1,68 @@
+"""The self-attention value-gradient scatter by query tiles (csrc/td_backward.hip, scatter_tile_kernel)."""
+
+import pytest
+import torch
+
+from inputs import workload
+from marearts_tinydeform_amd import _native
+from oracle import gridsample
+from test_gpu_backward import NAMES, check, gpu_grads, grad_out_for
+
+pytestmark = pytest.mark.gpu
+
+# B, H, D, P, levels: 16 x 16 tiles (131072 rows and more, 1024 threads) with maps that end inside a tile; 16 x 8, and
+# by P or D 8 x 8 and 8 x 4; five levels (the samples of four are loaded together); one map smaller than a tile
+SHAPES = [
+    (4, 8, 32, 4, [(55, 57), (28, 29), (14, 15)]),
+    (2, 8, 64, 8, [(65, 67), (61, 66)]),
+    (1, 2, 32, 4, [(33, 49), (17, 25), (9, 13), (5, 7), (3, 4)]),
+    (1, 2, 64, 4, [(31, 47), (16, 24)]),
+    (2, 2, 16, 16, [(24, 39)]),
+    (1, 4, 8, 2, [(9, 5), (40, 3)]),
+]
+
+
+@pytest.mark.parametrize('shape', SHAPES)
+@pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
+def test_tile_scatter(shape, dtype):
+    B, H, D, P, levels = shape
+    N = sum(h * w for h, w in levels)
+    args = workload(B, N, H, D, 64, levels, P, dtype, loc_dist='encoder', seed=5)
+    loc = args[5]
+    loc[:, ::7, :, :, 0] = 0.5              # many corners in one pixel, far from most of their tiles
+    loc[:, 3::11, :, :, -1] += 3.0          # outside the map
+    loc[:, 5::13, :, :, -1] = float('nan')
+    go = grad_out_for(args)
+    grads, _ = gpu_grads(args, go, dtype)
+    loc64 = loc.clone()
+    loc64[loc64.isnan()] = -9.0             # nothing, as a location outside
+    args[5] = loc64
+    ref = gridsample.deform_attn_grads(*args, go.to(dtype))
+    for n in NAMES:
+        check(f'tiles {shape} {dtype} d{n}', grads[n], ref[n], dtype)
+
+
+def test_tile_scatter_keeps_infinities_where_they_belong():
+    # an infinite grad_out row reaches the pixels it samples and no other, in float16 too
+    levels = [(20, 30), (10, 15)]
+    N = sum(h * w for h, w in levels)
+    args = workload(1, N, 2, 32, 64, levels, 4, torch.float16, loc_dist='encoder', seed=2)
+    # corners of non-zero weight only (0 times infinity is NaN, here as anywhere)
+    args[5][0, 100] = torch.linspace(0.2131, 0.4377, 2 * 2 * 4 * 2).view(2, 2, 4, 2).half()
+    for l, (h, w) in enumerate(levels):
+        pix = args[5][0, 100, :, l].float() * torch.tensor([w, h]) - 0.5
+        assert (pix != pix.floor()).all()
+    value = torch.randn(1, N, 64, generator=torch.Generator().manual_seed(1)).half()
+    go = torch.ones(1, N, 64).half()
+    go[0, 100, :32] = float('inf')          # head 0 of query 100
+    dev = [t.cuda() for t in (value, args[3], args[4], args[5], args[6])]
+    gv, _, _ = _native.sample_backward(dev[0], 2, dev[1], dev[2], dev[3], dev[4], go.cuda())
+    bad = (~gv.isfinite()).any(-1)[0].cpu()
+    assert torch.isfinite(gv[0, :, 32:]).all()
+    go[0, 100, :32] = 0
+    go[0, :100] = 0
+    go[0, 101:] = 0
+    go[0, 100, :32] = 1
+    alone, _, _ = _native.sample_backward(dev[0], 2, dev[1], dev[2], dev[3], dev[4], go.cuda())
+    hit = (alone[0, :, :32] != 0).any(-1).cpu()
+    assert hit.any() and bool((bad == hit).all())
