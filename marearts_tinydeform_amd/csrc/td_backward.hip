@@ -16,6 +16,7 @@
 // guard band has all four corners outside, so its gradient is 0, as for grid_sample's zero padding. Discrete
 // sampling (D-FINE) is piecewise constant in the location: its location gradient is 0.
 #include "td_gemm_mfma.h"
+#include "td_split.h"
 
 namespace td {
 namespace {
@@ -2059,6 +2060,110 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradParams p, int per_xcd) 
     wgrad_tile<T, VEC, TW>(p, idx, reinterpret_cast<T*>(lds), reinterpret_cast<T*>(lds + wgrad_slice_bytes<T>()));
 }
 
+// The weight gradient of float32 operands on the bfloat16 matrix units (td_split.h): the same tiles, splits and partials,
+// in steps of 32 tokens. Each thread takes 4 tokens x 4 columns of each operand, turns and splits them in registers,
+// and stores 8 bytes (4 tokens) a column and part; the next step's are loaded during the MFMAs, and two workgroups
+// share a CU, so that one splits while the other's MFMAs run. A step with values beyond the split is added by float32
+// FMAs. Against the float32 units (us, with the reduce): 67200 x 256 x 256 123.8 -> 80.5, 16800 47.1 -> 36.0, 20000 x
+// 512 x 512 138.5 -> 86.1, 21760 x 1024 x 1024 501.8 -> 301.5 (0.91 PFLOP/s of bfloat16 products; what is left beside
+// the MFMAs are a step's split, its two barriers and the loads behind them).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_split_kernel(WgradParams p,
+                                                                                                  int per_xcd) {
+    __shared__ __align__(16) SplitSlices s;
+    const int idx = static_cast<int>(blockIdx.x % kXcds) * per_xcd + static_cast<int>(blockIdx.x / kXcds);
+    const int tiles = p.nt * p.ct;
+    if (idx >= tiles * p.splits) return;  // the last XCD's spare workgroups
+    const int sp = idx / tiles, tile = idx - sp * tiles;
+    const int n0 = (tile / p.ct) * kSplitTile, c0 = (tile % p.ct) * kSplitTile;
+    const int m_begin = sp * p.chunk, m_end = min(p.M, m_begin + p.chunk);
+    const float* __restrict__ G = static_cast<const float*>(p.G);
+    const float* __restrict__ X = static_cast<const float*>(p.X);
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
+    const int wa = wave >> 1, wb = wave & 1, r = lane & 15, kg = lane >> 4;
+    const int tq = tid & 7, cb = (tid >> 3) * 4;  // this thread's tokens 4 tq .. + 3 of a step and columns cb .. + 3
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+    f32x4 pg[4], px[4], bsum = zero;
+    const bool gcol = n0 + cb < p.NO, xcol = c0 + cb < p.K, do_b = c0 == 0;
+    auto load = [&](int m0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int m = m0 + 4 * tq + u;
+            pg[u] = m < m_end && gcol ? *reinterpret_cast<const f32x4*>(G + static_cast<int64_t>(m) * p.NO + n0 + cb) : zero;
+            px[u] = m < m_end && xcol ? *reinterpret_cast<const f32x4*>(X + static_cast<int64_t>(m) * p.K + c0 + cb) : zero;
+        }
+    };
+    bool beyond = false;
+    auto stage = [&](const f32x4 (&v)[4], bf16* to) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const f32x4 col = {v[0][e], v[1][e], v[2][e], v[3][e]};
+            bf16x4 part[3];
+            split3(col, part[0], part[1], part[2]);
+            beyond |= beyond_split(col);
+            bf16* const at = to + split_at(cb + e, tq >> 1) + (tq & 1) * 4;
+#pragma unroll
+            for (int o = 0; o < 3; ++o) *reinterpret_cast<bf16x4*>(at + o * kSplitPlane) = part[o];
+        }
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = zero;
+    load(m_begin);
+    for (int m0 = m_begin; m0 < m_end; m0 += 32) {
+        beyond = false;
+        stage(pg, s.a);
+        stage(px, s.b);
+        if (do_b) bsum += (pg[0] + pg[1]) + (pg[2] + pg[3]);
+        const bool any = __any(beyond);
+        if (lane == 0) s.flags[wave] = any;
+        __syncthreads();
+        if (m0 + 32 < m_end) load(m0 + 32);  // in flight during this step's MFMAs
+        if (s.flags[0] | s.flags[1] | s.flags[2] | s.flags[3]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int n = n0 + 64 * wa + 16 * i + 4 * kg + e, c = c0 + 64 * wb + 16 * j + r;
+                        if (n >= p.NO || c >= p.K) continue;
+#pragma unroll 1
+                        for (int m = m0; m < min(m0 + 32, m_end); ++m)
+                            acc[i][j][e] = fmaf(G[static_cast<int64_t>(m) * p.NO + n],
+                                                X[static_cast<int64_t>(m) * p.K + c], acc[i][j][e]);
+                    }
+        } else {
+            split_mma(s, wa, wb, lane, acc);
+        }
+        __syncthreads();
+    }
+    float* part = p.part + static_cast<int64_t>(sp) * p.NO * p.K;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int c = c0 + 64 * wb + 16 * j + r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = n0 + 64 * wa + 16 * i + 4 * kg + e;
+                if (n < p.NO && c < p.K) part[static_cast<int64_t>(n) * p.K + c] = acc[i][j][e];
+            }
+        }
+    if (do_b) {  // the 8 lanes of a column group hold its tokens' sums
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v = bsum[e];
+            v += xor_lane(v, 1);
+            v += xor_lane(v, 2);
+            v += xor_lane(v, 4);
+            if (tq == 0 && n0 + cb + e < p.NO) p.bpart[static_cast<int64_t>(sp) * p.NO + n0 + cb + e] = v;
+        }
+    }
+}
+
 // The input gradient's GEMM (grad_memory = G . W, on the 64 x 64 two-stage tiles the value projection's size rule
 // picks below about 14000 tokens of 256 channels) and the weight gradient in one launch: they read the same G and
 // nothing of each other, and each alone leaves most of the GPU idle at those sizes (about 500 and 260 workgroups of
@@ -2495,10 +2600,16 @@ int launch_transpose(int dtype, const void* src, void* dst, int64_t R, int64_t C
     return launched("transpose");
 }
 
+// Whether the weight gradient of these operands runs on the split kernel: float32 with whole, aligned 16-byte rows.
+static bool wgrad_split_pays(int dtype, const void* G, const void* X, int64_t M, int64_t NO, int64_t K) {
+    return dtype == kF32 && split_size_pays(M, K) && NO % 4 == 0 && K % 4 == 0 &&
+           ((reinterpret_cast<uintptr_t>(G) | reinterpret_cast<uintptr_t>(X)) % 16) == 0;
+}
+
 // grad_memory = G . W (through W^T, as td_input_grad computes it) and the weight gradient of the same G: where the
 // value projection's size rule picks the 64 x 64 two-stage tiles for the input gradient, its tiles and the weight
-// gradient's run in one launch (input_weight_grad_kernel), except in float32 where the split kernel is the faster one
-// for the input gradient; otherwise the two run one after the other. The workspace
+// gradient's run in one launch (input_weight_grad_kernel), except in float32 where the split kernels take them;
+// otherwise the two run one after the other. The workspace
 // is the weight gradient's (td_weight_grad_workspace). M, HD and C are positive.
 int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, const void* X, void* gm, void* gw,
                              void* gb, int64_t M, int64_t HD, int64_t C, void* workspace, int64_t ws_bytes,
@@ -2506,12 +2617,12 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
     // grad_memory = G . W with W read as stored
     const GemmParams sp{G, W, nullptr, gm, static_cast<int>(M), static_cast<int>(HD), static_cast<int>(C), 0, 0, 0};
     int rc = 0;
-    if (dtype == kF32 && gemm_split_pays(sp)) {
+    if (dtype == kF32 && gemm_split_pays(sp) && wgrad_split_pays(dtype, G, X, M, HD, C)) {
         rc = launch_gemm_split(sp, stream, true);
         if (rc != 0) return rc;
         return launch_wgrad(dtype, G, X, gw, gb, M, HD, C, workspace, ws_bytes, stream);
     }
-    if (value_proj_plan(dtype, G, Wt, nullptr, gm, M, HD, C, 0, 0) == 25) {
+    if (value_proj_plan(dtype, G, Wt, nullptr, gm, M, HD, C, 0, 0) == 25 && !wgrad_split_pays(dtype, G, X, M, HD, C)) {
         // 16-bit with C a multiple of 8 and W 16-byte aligned: the GEMM reads W as stored (no transpose launch,
         // Wt is left unwritten)
         const bool stored = (dtype == kF16 || dtype == kBF16) && C % 8 == 0 &&
@@ -2542,7 +2653,9 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
 // B8 124.6 -> 129.0 (half the tiles, so twice the splits and partials)
 constexpr int64_t kWgWideMinK = 512;
 
-int wgrad_width(int64_t K, int dtype) { return dtype != kF64 && K >= kWgWideMinK ? 2 : 1; }
+int wgrad_width(int64_t M, int64_t K, int dtype) {
+    return dtype != kF64 && K >= kWgWideMinK && !(dtype == kF32 && split_size_pays(M, K)) ? 2 : 1;
+}
 
 // Split count of the weight gradient: about 512 workgroups (1024 for large outputs), at least four token steps per
 // split (64 tokens in float32, 128 otherwise). Measured on the training step at 8400 tokens (256 x 256), against 256
@@ -2550,7 +2663,7 @@ int wgrad_width(int64_t K, int dtype) { return dtype != kF64 && K >= kWgWideMinK
 // (63.4 with 64); problems of 32768 tokens and more already had their 512 workgroups.
 static void wgrad_split(int64_t M, int64_t NO, int64_t K, int dtype, int tw, int* splits, int* chunk) {
     const int64_t tiles = ((NO + kWgTile - 1) / kWgTile) * ((K + tw * kWgTile - 1) / (tw * kWgTile));
-    const int kb = dtype == kF32 ? 16 : 32;
+    const int kb = dtype == kF32 && !split_size_pays(M, K) ? 16 : 32;
     // 1024 workgroups from 64 output tiles (C = 1024): training step at C = 1024 bf16 B2 Q300 913.0 -> 895.2 us; at
     // 4 tiles (C = 256) 1024 lost 1.5-5% (DINO B4 Q900, bf16 B8 Q300, the DINO encoder: more partials to reduce)
     const int64_t target = tiles >= 64 ? 1024 : 512;
@@ -2575,7 +2688,7 @@ static void wgrad_split(int64_t M, int64_t NO, int64_t K, int dtype, int tw, int
 void wgrad_plan(int64_t M, int64_t NO, int64_t K, int dtype, int* splits, int* chunk, int64_t* ws_bytes) {
     int s1 = 1, c1 = 32;
     wgrad_split(M, NO, K, dtype, 1, &s1, &c1);
-    const int tw = wgrad_width(K, dtype);
+    const int tw = wgrad_width(M, K, dtype);
     *splits = s1;
     *chunk = c1;
     if (tw != 1) wgrad_split(M, NO, K, dtype, tw, splits, chunk);
@@ -2592,8 +2705,8 @@ int launch_wgrad(int dtype, const void* G, const void* X, void* gw, void* gb, in
         return set_error(-4, "weight gradient: workspace of %lld bytes needed, %lld given", static_cast<long long>(need),
                          static_cast<long long>(ws_bytes));
     if (NO * K == 0) return 0;
-    const int tw = with_gemm != nullptr ? 1 : wgrad_width(K, dtype);
-    if (tw != wgrad_width(K, dtype)) wgrad_split(M, NO, K, dtype, tw, &splits, &chunk);
+    const int tw = with_gemm != nullptr ? 1 : wgrad_width(M, K, dtype);
+    if (tw != wgrad_width(M, K, dtype)) wgrad_split(M, NO, K, dtype, tw, &splits, &chunk);
     WgradParams p{G, X, nullptr, nullptr, static_cast<int>(M), static_cast<int>(NO), static_cast<int>(K),
                   static_cast<int>((NO + kWgTile - 1) / kWgTile),
                   static_cast<int>((K + tw * kWgTile - 1) / (tw * kWgTile)), splits, chunk};
@@ -2624,7 +2737,11 @@ int launch_wgrad(int dtype, const void* G, const void* X, void* gw, void* gb, in
     const int E = dtype == kF32 ? 4 : 8;
     const bool vec = NO % E == 0 && K % E == 0 &&
                      ((reinterpret_cast<uintptr_t>(G) | reinterpret_cast<uintptr_t>(X)) % 16) == 0;
-    if (with_gemm != nullptr) {
+    if (wgrad_split_pays(dtype, G, X, M, NO, K)) {
+        const int per_xcd = static_cast<int>((static_cast<int64_t>(grid.x) + kXcds - 1) / kXcds);
+        hipLaunchKernelGGL(wgrad_split_kernel, dim3(static_cast<unsigned>(per_xcd * kXcds)), dim3(256), 0, stream, p,
+                           per_xcd);
+    } else if (with_gemm != nullptr) {
         // the input gradient's GEMM tiles first, numbered as its own launch numbers them, then the weight gradient's
         GemmParams gp = *with_gemm;
         gp.mt = (gp.M + 63) / 64;

@@ -91,6 +91,12 @@ int launch_gemm_stream(int dtype, GemmParams p, hipStream_t stream, bool w_store
 
 // Its float32 counterpart on split operands (td_gemm_split.hip): NO = 256, K = 128 or 256, row-major output, 16-byte
 // aligned a, w and c (gemm_split_fits); gemm_split_pays also asks for the rows from which it is the faster kernel.
+// Sizes (rows x channels) from which float32 products are faster split: 6400 rows of 256 channels. Projection K = 256:
+// 5000 rows 13.4 us against 12.1 split, 8400 19.8 against 15.4, 2400 8.8 against 11.7 (the split kernel's start is 8
+// of them); both projection gradients, K = 256: 5000 rows 35.9 in the combined launch against 38.0, 8400 51.9 against
+// 47.5; 8400 x 384 84.7 against 73.1, 6000 x 512 106.6 against 82.0, 5000 x 128 21.9 against 27.5. One line for the
+// three products, so that each has the same bits whichever entry computes it.
+inline bool split_size_pays(int64_t M, int64_t K) { return M >= 2048 && M * K >= 6400 * 256; }
 bool gemm_split_fits(const GemmParams& p);
 bool gemm_split_pays(const GemmParams& p);
 int launch_gemm_split(GemmParams p, hipStream_t stream, bool w_stored = false);

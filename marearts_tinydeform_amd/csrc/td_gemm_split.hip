@@ -308,9 +308,7 @@ bool gemm_split_fits(const GemmParams& p) {
     return p.NO == kSplitNO && (p.K == 128 || p.K == 256) && p.M > 0 && al % 16 == 0 && p.hm_D == 0;
 }
 
-// From 4500 rows (the register tiles at 5000 rows: 13.4 us against 12.1 here, K = 128 9.0 against 8.1; at 2400 rows 8.8
-// against 11.7, the start being 8 of them)
-bool gemm_split_pays(const GemmParams& p) { return p.M >= 4500 && gemm_split_fits(p); }
+bool gemm_split_pays(const GemmParams& p) { return split_size_pays(p.M, p.K) && gemm_split_fits(p); }
 
 int launch_gemm_split(GemmParams p, hipStream_t stream, bool w_stored) {
     if (!gemm_split_fits(p)) return set_error(-1, "value_proj: the split kernel does not take this shape");

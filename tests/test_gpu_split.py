@@ -21,9 +21,9 @@ def problem(M, K, NO, seed=0):
     return x, w, torch.randn(NO, generator=g)
 
 
-# one row past 4500 (one step of 18 tokens a workgroup), shares that end 1 and 16 and 17 tokens into a step, many steps
-@pytest.mark.parametrize('M', [4501, 8193, 12288, 12545, 33600, 67201])
-@pytest.mark.parametrize('K', [128, 256])
+# one step a workgroup, shares that end 1, 16 and 17 tokens into a step, many steps
+@pytest.mark.parametrize('M,K', [(6401, 256), (8193, 256), (12288, 256), (12545, 256), (67201, 256), (12801, 128),
+                                 (16385, 128), (33600, 128), (45057, 128)])
 @pytest.mark.parametrize('bias', [True, False])
 def test_split_projection(M, K, bias):
     x, w, b = problem(M, K, 256)
@@ -38,7 +38,8 @@ def test_split_projection(M, K, bias):
 @pytest.mark.parametrize('K', [128, 256])
 def test_split_projection_beyond_the_split(K):
     # infinities, NaN and values whose bfloat16 rounds to infinity: what float32 arithmetic gives, and only there
-    x, w, _ = problem(9001, K, 256)
+    M = 2304001 // K  # 9000 rows of 256
+    x, w, _ = problem(M, K, 256)
     x[0, 40, 3], x[0, 41, 5], x[0, 8999, 0], x[0, 77, 1] = float('inf'), float('nan'), -float('inf'), 3.4e38
     w[7, 1] = 0.0
     got = _native.value_proj(x.cuda(), w.cuda(), None).cpu()
@@ -47,7 +48,7 @@ def test_split_projection_beyond_the_split(K):
     assert torch.equal(got[0, rows].isnan(), ref[0, rows].isnan())
     assert torch.equal(got[0, rows].nan_to_num(0, 1, -1), ref[0, rows].nan_to_num(0, 1, -1))
     assert torch.allclose(got[0, 77], ref[0, 77], rtol=1e-5, atol=0) and got[0, 77, 7].abs() < 100
-    keep = torch.ones(9001, dtype=torch.bool)
+    keep = torch.ones(M, dtype=torch.bool)
     keep[rows + [77]] = False
     assert torch.allclose(got[0, keep], ref[0, keep], rtol=0, atol=2e-5)
     # a weight beyond the split reaches every token
@@ -69,7 +70,34 @@ def test_split_input_gradient():
 
 def test_split_projection_of_unaligned_rows():
     # operands off a 16-byte boundary keep the kernels that take them
-    x, w, b = problem(5000, 256, 256)
+    x, w, b = problem(7000, 256, 256)
     got = _native.value_proj(shifted(x.cuda(), 4), w.cuda(), b.cuda()).cpu().double()
     ref = torch.from_numpy(bruteforce.project(x, w, b))
     assert (got - ref).abs().max() < 1e-4
+
+
+# tiles cut on both sides, one partial split, many; bias in the last, partial, tile of columns
+@pytest.mark.parametrize('M,NO,K', [(6401, 256, 256), (20011, 256, 128), (4801, 384, 384), (9001, 100, 260),
+                                    (16003, 132, 200), (2048, 64, 1024)])
+def test_split_weight_gradient(M, NO, K):
+    gen = torch.Generator().manual_seed(1)
+    G, X = torch.randn(1, M, NO, generator=gen), torch.randn(1, M, K, generator=gen)
+    gw, gb = _native.weight_grad(G.cuda(), X.cuda())
+    G64, X64 = G[0].double(), X[0].double()
+    # sums over M tokens in splits: the largest sum's roundings, as above
+    assert ((gw.cpu().double() - G64.T @ X64).abs() <= M ** 0.5 * 8 * EPS * (G64.abs().T @ X64.abs()) / M ** 0.5).all()
+    assert ((gb.cpu().double() - G64.sum(0)).abs() <= 64 * EPS * G64.abs().sum(0)).all()
+
+
+def test_split_weight_gradient_beyond_the_split():
+    G, X = torch.randn(1, 8192, 256), torch.randn(1, 8192, 256)
+    G[0, 5, 7], X[0, 900, 3], G[0, 3000, 9] = float('inf'), float('nan'), 3.3e38
+    gw, _ = _native.weight_grad(G.cuda(), X.cuda())
+    gw = gw.cpu()
+    ref = G[0].double().T @ X[0].double()
+    assert gw[:, 3].isnan().all() and not gw[:7, [0, 1, 2]].isnan().any()
+    rest = [c for c in range(256) if c != 3]
+    assert torch.equal(gw[7, rest], torch.full((255,), float('inf')) * X[0, 5, rest].sign())
+    over = ref[9, rest].abs() > 3.4e38
+    assert torch.equal(gw[9, rest].isinf(), over) or ((gw[9, rest].isinf() == over) | (ref[9, rest].abs() > 3.39e38)).all()
+    assert torch.allclose(gw[10:, rest].double(), ref[10:, rest], rtol=0, atol=2e-3)
