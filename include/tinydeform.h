@@ -35,6 +35,7 @@ extern "C" {
 #define TD_F16 1
 #define TD_BF16 2
 #define TD_F64 3
+#define TD_ACC_SCRATCH 16 /* td_sample_backward, with TD_F32: grad_value_acc is scratch */
 
 /* error codes */
 #define TD_OK 0
@@ -260,7 +261,9 @@ int td_sample_plan(int dtype, int64_t B, int64_t Q, int64_t N, int64_t H, int64_
  *                               TD_F32 / TD_F64). For TD_F16 / TD_BF16 with grad_value given, decoder shapes with
  *                               many corners (2^18 or more) may have grad_value written directly, by binning the
  *                               corners by token, with grad_value_acc used as scratch only: its contents are then
- *                               unspecified, so read the value gradient from grad_value;
+ *                               unspecified, so read the value gradient from grad_value. dtype TD_F32 |
+ *                               TD_ACC_SCRATCH lets float32 do the same (grad_value then given, and not
+ *                               grad_value_acc itself);
  *   grad_loc [B, Q, H, L, P, 2], grad_attn [B, Q, H, L, P]: dtype.
  * padding_mask as in td_sample_forward_masked. Limits as td_sample_forward, and D <= 256.
  */

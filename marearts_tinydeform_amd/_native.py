@@ -51,6 +51,7 @@ SIGNATURES = {
     'td_probe_atomic': (_int, [_vp, _i64, _i64, _i64, _i64, _int, _vp]),
 }
 
+ACC_SCRATCH = 16  # TD_ACC_SCRATCH
 TD_E_WORKSPACE = -4  # td_layer_fused_forward: the problem needs loc_out / attn_out
 
 load_error = None
@@ -461,12 +462,16 @@ def sample_backward(value, heads, spatial_shapes, level_start_index, sampling_lo
     lc, aw = sampling_locations.contiguous(), attention_weights.contiguous()
     sh, st = spatial_shapes.contiguous(), level_start_index.contiguous()
     acc = torch.empty((B, N, HD), dtype=acc_dtype(dt), device=dev)
-    gv = acc if acc.dtype == dt else torch.empty((B, N, HD), dtype=dt, device=dev)
+    # float32 (float64) sums are the gradient; from 2^18 corners on a float32 decoder's are binned in the accumulator's
+    # memory and written beside it
+    binned = dt == torch.float32 and B * Q * H * L * P * 4 >= 1 << 18 and Q * L * P * 4 < 16 * N
+    gv = acc if acc.dtype == dt and not binned else torch.empty((B, N, HD), dtype=dt, device=dev)
     gl = torch.empty_like(lc)
     ga = torch.empty_like(aw)
     if acc.numel() == 0 and gl.numel() == 0:
         return gv, gl, ga
-    _check(lib_.td_sample_backward(DTYPE_CODES[dt], v.data_ptr(), sh.data_ptr(), st.data_ptr(), lc.data_ptr(),
+    code = DTYPE_CODES[dt] | (ACC_SCRATCH if binned else 0)
+    _check(lib_.td_sample_backward(code, v.data_ptr(), sh.data_ptr(), st.data_ptr(), lc.data_ptr(),
                                    aw.data_ptr(), _ptr(mask), go.data_ptr(), acc.data_ptr(), gv.data_ptr(),
                                    gl.data_ptr(), ga.data_ptr(), B, Q, N, H, HD // H, L, P, _stream(dev)))
     return gv, gl, ga

@@ -540,6 +540,8 @@ extern "C" int td_sample_backward(int dtype, const void* value, const int64_t* s
                                   const void* attention_weights, const uint8_t* padding_mask, const void* grad_out,
                                   void* grad_value_acc, void* grad_value, void* grad_loc, void* grad_attn, int64_t B,
                                   int64_t Q, int64_t N, int64_t H, int64_t D, int64_t L, int64_t P, void* stream) {
+    const bool acc_scratch = dtype == (TD_F32 | TD_ACC_SCRATCH);
+    if (acc_scratch) dtype = TD_F32;
     int rc = check_geometry(dtype, B, Q, N, H, D, L, P, spatial_shapes, level_start_index, sampling_locations,
                             attention_weights, grad_loc);
     if (rc != TD_OK) return rc;
@@ -554,7 +556,8 @@ extern "C" int td_sample_backward(int dtype, const void* value, const int64_t* s
     const hipStream_t s = static_cast<hipStream_t>(stream);
     bool direct = false;
     rc = launch_sample_backward(dtype, value, g, sampling_locations, attention_weights, grad_out, grad_value_acc,
-                                grad_value == grad_value_acc ? nullptr : grad_value, grad_loc, grad_attn, s, &direct);
+                                grad_value == grad_value_acc ? nullptr : grad_value, grad_loc, grad_attn, s, &direct,
+                                acc_scratch);
     if (rc != TD_OK || direct || grad_value == nullptr || grad_value == grad_value_acc) return rc;
     return launch_convert(dtype, grad_value_acc, grad_value, B * N * H * D, s);
 }

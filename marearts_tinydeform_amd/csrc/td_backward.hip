@@ -1347,7 +1347,7 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
     }
 }
 
-// The value gradient by binning the corners by token (decoder shapes, 16-bit types). With few corner hits per token
+// The value gradient by binning the corners by token (decoder shapes, 16- and 32-bit types). With few corner hits per token
 // (decoders: 2-4 per token and head) the atomic scatter runs at the GPU's float-atomic rate (about 320 G lane-adds/s,
 // one 128-byte line per corner at D = 32) and needs a zeroed float32 accumulator and a rounding pass. LDS float
 // atomics are no way out: ds_add_f32 runs at about 0.33 lanes per clock per CU (about 200 G lane-adds/s over the GPU,
@@ -2410,9 +2410,9 @@ int loc_attn_backward_go(const BackParams& p, hipStream_t stream) {
     return launched("sample backward locations");
 }
 
-// The binned path (sort_count_kernel ... sort_reduce_kernel) for 16-bit types at decoder densities, with the location
-// and weight gradients from loc_attn_backward_kernel; grad_value (the element type, 8-byte aligned) is written
-// directly. Returns 1 without launching when it does not apply: too few corners to pay for its five launches, a dense
+// The binned path (sort_count_kernel ... sort_reduce_kernel) at decoder densities, with the location and weight
+// gradients from loc_attn_backward_kernel; grad_value (the element type, aligned to four elements, not the
+// accumulator) is written directly. Returns 1 without launching when it does not apply: too few corners to pay for its five launches, a dense
 // problem (the bucketed scatter's), a head width other than 8..64 (a power of two), more than kSortMaxBins bins or
 // 2^25 rows, scratch that does not fit in the accumulator buffer (acc_bytes), or shapes loc_attn_backward_kernel
 // does not take (value or grad_out rows not 16-byte aligned).
@@ -2421,7 +2421,7 @@ constexpr int64_t kSortMinCorners = int64_t{1} << 18;
 template <typename T>
 int sample_backward_sorted(const BackParams& p, void* grad_value_t, int64_t acc_bytes, hipStream_t stream) {
     const Geom& g = p.g;
-    if (grad_value_t == nullptr || grad_value_t == p.grad_value || reinterpret_cast<uintptr_t>(grad_value_t) % 8 != 0 ||
+    if (grad_value_t == nullptr || grad_value_t == p.grad_value || reinterpret_cast<uintptr_t>(grad_value_t) % (4 * sizeof(T)) != 0 ||
         reinterpret_cast<uintptr_t>(p.grad_value) % 16 != 0 || !is_pow2(g.D) || g.D < 8 || g.D > 64 || g.LP <= 0 ||
         g.LP > 256 || g.L > kMaxLevelPoints || bucket_scatter_pays(g))
         return 1;
@@ -2524,21 +2524,27 @@ int sample_backward_t(const BackParams& p, hipStream_t stream) {
 
 int launch_sample_backward(int dtype, const void* value, const Geom& g, const void* loc, const void* attn,
                            const void* grad_out, void* grad_value, void* grad_value_t, void* grad_loc, void* grad_attn,
-                           hipStream_t stream, bool* direct) {
+                           hipStream_t stream, bool* direct, bool acc_scratch) {
     if (g.D > kWave * 4) return set_error(-1, "sample backward: head dim %d > %d", g.D, kWave * 4);
     const int acc = dtype == kF64 ? 8 : 4;
     const int64_t acc_bytes = static_cast<int64_t>(g.B) * g.N * g.H * g.D * acc;
     BackParams p{value, loc, attn, grad_out, grad_value, grad_loc, grad_attn, g, 1};
     *direct = false;
-    if ((dtype == kF16 || dtype == kBF16) && (reinterpret_cast<uintptr_t>(grad_value) % 8) == 0) {
-        const int rs = dtype == kF16 ? sample_backward_sorted<f16>(p, grad_value_t, acc_bytes, stream)
-                                     : sample_backward_sorted<bf16>(p, grad_value_t, acc_bytes, stream);
+    if (dtype != kF64 && (reinterpret_cast<uintptr_t>(grad_value) % 8) == 0) {
+        const int rs = dtype == kF32   ? sample_backward_sorted<float>(p, acc_scratch ? grad_value_t : nullptr, acc_bytes,
+                                                                        stream)
+                       : dtype == kF16 ? sample_backward_sorted<f16>(p, grad_value_t, acc_bytes, stream)
+                                       : sample_backward_sorted<bf16>(p, grad_value_t, acc_bytes, stream);
         if (rs != 1) {
             *direct = rs == 0;
             return rs;
         }
     }
-    const int rc = launch_zero(grad_value, acc_bytes, stream);
+    if (dtype == kF32 && acc_scratch && grad_value_t != nullptr) {  // no rounding to do: summed where it is wanted
+        p.grad_value = grad_value_t;
+        *direct = true;
+    }
+    const int rc = launch_zero(p.grad_value, acc_bytes, stream);
     if (rc != 0) return rc;
     switch (dtype) {
         case kF32: return sample_backward_t<float>(p, stream);
@@ -2653,9 +2659,7 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
 // B8 124.6 -> 129.0 (half the tiles, so twice the splits and partials)
 constexpr int64_t kWgWideMinK = 512;
 
-int wgrad_width(int64_t M, int64_t K, int dtype) {
-    return dtype != kF64 && K >= kWgWideMinK && !(dtype == kF32 && split_size_pays(M, K)) ? 2 : 1;
-}
+int wgrad_width(int64_t K, int dtype) { return dtype != kF64 && K >= kWgWideMinK ? 2 : 1; }
 
 // Split count of the weight gradient: about 512 workgroups (1024 for large outputs), at least four token steps per
 // split (64 tokens in float32, 128 otherwise). Measured on the training step at 8400 tokens (256 x 256), against 256
@@ -2663,7 +2667,7 @@ int wgrad_width(int64_t M, int64_t K, int dtype) {
 // (63.4 with 64); problems of 32768 tokens and more already had their 512 workgroups.
 static void wgrad_split(int64_t M, int64_t NO, int64_t K, int dtype, int tw, int* splits, int* chunk) {
     const int64_t tiles = ((NO + kWgTile - 1) / kWgTile) * ((K + tw * kWgTile - 1) / (tw * kWgTile));
-    const int kb = dtype == kF32 && !split_size_pays(M, K) ? 16 : 32;
+    const int kb = dtype == kF32 ? 16 : 32;
     // 1024 workgroups from 64 output tiles (C = 1024): training step at C = 1024 bf16 B2 Q300 913.0 -> 895.2 us; at
     // 4 tiles (C = 256) 1024 lost 1.5-5% (DINO B4 Q900, bf16 B8 Q300, the DINO encoder: more partials to reduce)
     const int64_t target = tiles >= 64 ? 1024 : 512;
@@ -2688,7 +2692,7 @@ static void wgrad_split(int64_t M, int64_t NO, int64_t K, int dtype, int tw, int
 void wgrad_plan(int64_t M, int64_t NO, int64_t K, int dtype, int* splits, int* chunk, int64_t* ws_bytes) {
     int s1 = 1, c1 = 32;
     wgrad_split(M, NO, K, dtype, 1, &s1, &c1);
-    const int tw = wgrad_width(M, K, dtype);
+    const int tw = wgrad_width(K, dtype);
     *splits = s1;
     *chunk = c1;
     if (tw != 1) wgrad_split(M, NO, K, dtype, tw, splits, chunk);
@@ -2705,8 +2709,13 @@ int launch_wgrad(int dtype, const void* G, const void* X, void* gw, void* gb, in
         return set_error(-4, "weight gradient: workspace of %lld bytes needed, %lld given", static_cast<long long>(need),
                          static_cast<long long>(ws_bytes));
     if (NO * K == 0) return 0;
-    const int tw = with_gemm != nullptr ? 1 : wgrad_width(M, K, dtype);
-    if (tw != wgrad_width(M, K, dtype)) wgrad_split(M, NO, K, dtype, tw, &splits, &chunk);
+    const bool split = wgrad_split_pays(dtype, G, X, M, NO, K);
+    const int tw = with_gemm != nullptr || split ? 1 : wgrad_width(K, dtype);
+    if (tw != wgrad_width(K, dtype)) wgrad_split(M, NO, K, dtype, tw, &splits, &chunk);
+    if (split) {  // whole steps of 32 tokens: at most the plan's splits
+        chunk = (chunk + 31) / 32 * 32;
+        splits = static_cast<int>((M + chunk - 1) / chunk);
+    }
     WgradParams p{G, X, nullptr, nullptr, static_cast<int>(M), static_cast<int>(NO), static_cast<int>(K),
                   static_cast<int>((NO + kWgTile - 1) / kWgTile),
                   static_cast<int>((K + tw * kWgTile - 1) / (tw * kWgTile)), splits, chunk};
@@ -2737,7 +2746,7 @@ int launch_wgrad(int dtype, const void* G, const void* X, void* gw, void* gb, in
     const int E = dtype == kF32 ? 4 : 8;
     const bool vec = NO % E == 0 && K % E == 0 &&
                      ((reinterpret_cast<uintptr_t>(G) | reinterpret_cast<uintptr_t>(X)) % 16) == 0;
-    if (wgrad_split_pays(dtype, G, X, M, NO, K)) {
+    if (split) {
         const int per_xcd = static_cast<int>((static_cast<int64_t>(grid.x) + kXcds - 1) / kXcds);
         hipLaunchKernelGGL(wgrad_split_kernel, dim3(static_cast<unsigned>(per_xcd * kXcds)), dim3(256), 0, stream, p,
                            per_xcd);

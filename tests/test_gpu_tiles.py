@@ -66,3 +66,32 @@ def test_tile_scatter_keeps_infinities_where_they_belong():
     alone, _, _ = _native.sample_backward(dev[0], 2, dev[1], dev[2], dev[3], dev[4], go.cuda())
     hit = (alone[0, :, :32] != 0).any(-1).cpu()
     assert hit.any() and bool((bad == hit).all())
+
+
+@pytest.mark.parametrize('D', [8, 16, 32, 64])
+@pytest.mark.parametrize('masked', [False, True])
+def test_binned_float32_value_gradient(D, masked):
+    # the decoders' binned value gradient in float32 (2^18 corners and more), hot spots and uniform locations in turn;
+    # and with the accumulator kept, which holds the gradient as it always did
+    levels, B, Q, H, P = [(40, 60), (20, 30), (10, 15)], 2, 350, 8, 4
+    N = sum(h * w for h, w in levels)
+    for where in ('clustered', 'uniform'):
+        args = workload(B, Q, H, D, 64, levels, P, torch.float32, loc_dist=where, seed=4)
+        args[5] = (args[5] * 4096).round() / 4096     # pixels that do not hang on how a product rounds
+        mask = torch.rand(B, N, generator=torch.Generator().manual_seed(4)) < 0.3 if masked else None
+        go = grad_out_for(args)
+        grads, _ = gpu_grads(args, go, torch.float32, mask=mask)
+        ref = gridsample.deform_attn_grads(*args, go, padding_mask=mask)
+        for n in NAMES:
+            check(f'binned float32 D={D} {where} d{n}', grads[n], ref[n], torch.float32)
+    value = torch.randn(B, N, H * D).cuda()
+    shapes, starts, loc, attn, go = (t.cuda() for t in (args[3], args[4], args[5], args[6], go))
+    gv, gl, ga = _native.sample_backward(value, H, shapes, starts, loc, attn, go)
+    acc, out = torch.empty_like(value), torch.empty_like(value)
+    gl2, ga2 = torch.empty_like(loc), torch.empty_like(attn)
+    rc = _native.lib.td_sample_backward(0, value.data_ptr(), shapes.data_ptr(), starts.data_ptr(), loc.data_ptr(),
+                                        attn.data_ptr(), None, go.data_ptr(), acc.data_ptr(), out.data_ptr(),
+                                        gl2.data_ptr(), ga2.data_ptr(), B, Q, N, H, D, len(levels), P,
+                                        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0 and torch.equal(acc, out)
+    assert torch.allclose(gv, acc, rtol=1e-4, atol=1e-4) and torch.allclose(ga, ga2, rtol=1e-4, atol=1e-4)
