@@ -7,6 +7,7 @@ libtinydeform.so; CPU tensors run the PyTorch reference path. Inference only.
 
 import functools
 import math
+import operator
 
 import torch
 
@@ -145,6 +146,15 @@ def cost_features(B, Q, H, D, C, N, L, P, s, aligned=True):
     return fused, gemm, sample
 
 
+@functools.lru_cache(maxsize=1024)
+def _features(B, Q, H, D, C, N, L, P, s, aligned):
+    """cost_features and gap_features of a problem's sizes, kept by those sizes: a model calls with a few over and over,
+    and the three plan calls and their arithmetic were 9 of an eager call's 24 us (the coefficients, which a caller may
+    replace, are applied each time)."""
+    return (*(tuple(f) for f in cost_features(B, Q, H, D, C, N, L, P, s, aligned)),
+            tuple(gap_features(B, Q, N, H, D, L, P, s)))
+
+
 # cost tables by GPU architecture (gcnArchName without feature suffixes)
 ARCH_LIMITS = {'gfx950': FUSED_LIMIT}
 
@@ -188,12 +198,12 @@ def _predict(memory, value_weight, Q, H, L, P, table=None):
     if isinstance(coef, tuple):
         raise ValueError('a threshold table (a, b) gives a mode, not times: use choose_mode')
     aligned = (memory.data_ptr() | value_weight.data_ptr()) % 16 == 0
-    ff, fg, fs = cost_features(B, Q, H, D, C, N, L, P, s, aligned)
+    ff, fg, fs, gap = _features(B, Q, H, D, C, N, L, P, s, aligned)
+
     def dot(c, x):
-        return sum(a * b for a, b in zip(c, x))
+        return sum(map(operator.mul, c, x))
     return {'fused': dot(coef['fused'], ff),
-            'project': dot(coef['gemm'], fg) + dot(coef['sample'], fs) +
-                       dot(coef['gap'], gap_features(B, Q, N, H, D, L, P, s))}
+            'project': dot(coef['gemm'], fg) + dot(coef['sample'], fs) + dot(coef['gap'], gap)}
 
 
 def choose_mode(memory, value_weight, sampling_locations):
