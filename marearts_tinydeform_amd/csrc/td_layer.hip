@@ -103,9 +103,9 @@ int finalize_prologue(const LayerArgs& la, const Geom& g, hipStream_t stream) {
 // into loc_out and attn_out) and the in-place finalize. A workgroup of the single-kernel prologue owns 16 queries of
 // one head and streams that head's weights once per 16 queries, so for large problems the weights are read
 // B * Q / 16 times; the GEMM tiles 64 queries x 64 outputs and keeps them in LDS. Returns 1, launching nothing,
-// when the GEMM cannot take the operands.
+// when the GEMM cannot take the operands (with pair_only: when both projections in one launch cannot).
 template <typename T>
-int launch_prologue_gemm(const LayerArgs& la, const Geom& g, hipStream_t stream) {
+int launch_prologue_gemm(const LayerArgs& la, const Geom& g, hipStream_t stream, bool pair_only) {
     constexpr int V = 16 / static_cast<int>(sizeof(T));
     const uintptr_t al = reinterpret_cast<uintptr_t>(la.query) | reinterpret_cast<uintptr_t>(la.pos) |
                          reinterpret_cast<uintptr_t>(la.off_w) | reinterpret_cast<uintptr_t>(la.aw_w) |
@@ -118,6 +118,7 @@ int launch_prologue_gemm(const LayerArgs& la, const Geom& g, hipStream_t stream)
     if (rc < 0) return rc;
     if (rc == 2) return 0;  // finalized in the projections' epilogue
     if (rc == 0) return finalize_prologue<T>(la, g, stream);
+    if (pair_only) return 1;
     rc = launch_proj_f32(dt, la.query, la.pos, la.off_w, la.off_b, static_cast<float*>(la.loc_out), M, la.Cq, 2 * NO,
                          stream);
     if (rc != 0) return rc;
@@ -175,15 +176,22 @@ bool prologue_wants_gemm(int dtype, const Geom& g, int64_t Cq) {
 int launch_prologue(int dtype, const LayerArgs& layer, const Geom& g, hipStream_t stream, int route) {
     if (layer.loc_out == nullptr || layer.attn_out == nullptr)
         return set_error(-1, "layer prologue: locations and weights need output buffers");
-    // route 0: by the projections' multiply-adds. Measured on MI355X: the single kernel up to DINO-sized problems
-    // (3600 queries, Cq 256, 8 heads x 16 samples, 3.5e8: 14-17 µs against 25 µs for the GEMM route), the GEMM route
-    // for the C = 1024 shape (600 queries, 16 heads x 64 samples, 1.9e9: 45 µs against 72 µs).
-    if (dtype != kF64 && (route == 2 || (route == 0 && prologue_wants_gemm(dtype, g, layer.Cq)))) {
+    // route 0: by the projections' multiply-adds. In 16 bits, where both projections share a launch (gemm_pair_kernel)
+    // and mostly the finalize too, the GEMM route from 1.2e8 (us, single kernel against GEMM route): fp16 C = 256, 8
+    // heads x 16 samples: 900 queries (0.9e8) 7.6 against 7.9, 1800 10.2 / 8.2, 3600 15.9 / 8.8, 7200 24.8 / 13.3; 8
+    // heads x 12 samples: 2100 10.2 / 9.3, 7200 22.0 / 18.2; C = 512 300 queries (1.2e8) 10.0 / 9.3, 1200 19.1 / 9.7;
+    // C = 1024 300 queries 15.5 / 12.0. With two launches and a finalize of its own (other types and sizes) from 8e8
+    // (600 queries, 16 heads x 64 samples, 1.9e9: 45 against 72).
+    const double macs = static_cast<double>(g.B) * g.Q * g.H * 3 * g.LP * layer.Cq;
+    const bool large = prologue_wants_gemm(dtype, g, layer.Cq);
+    const bool pair = (dtype == kF16 || dtype == kBF16) && macs >= 1.2e8;
+    if (dtype != kF64 && (route == 2 || (route == 0 && (large || pair)))) {
+        const bool pair_only = route == 0 && !large;
         int rc = 1;
         switch (dtype) {
-            case kF32: rc = launch_prologue_gemm<float>(layer, g, stream); break;
-            case kF16: rc = launch_prologue_gemm<f16>(layer, g, stream); break;
-            case kBF16: rc = launch_prologue_gemm<bf16>(layer, g, stream); break;
+            case kF32: rc = launch_prologue_gemm<float>(layer, g, stream, pair_only); break;
+            case kF16: rc = launch_prologue_gemm<f16>(layer, g, stream, pair_only); break;
+            case kBF16: rc = launch_prologue_gemm<bf16>(layer, g, stream, pair_only); break;
             default: break;
         }
         if (rc <= 0) return rc;  // launched, or failed; 1: the GEMM cannot take the operands
