@@ -121,6 +121,8 @@ def cost_features(B, Q, H, D, C, N, L, P, s, aligned=True):
     split = s == 4 and v > 0 and NO == 256 and K in (128, 256) and M * K >= 6400 * 256 and not hm  # float32 on split operands
     if v == 22 or split:
         gemm[1] = -(-(-(-M // CUS)) // 32) * 32 * (K + NO) * s * CUS / 1e6
+        if s == 2 and K == 384:  # its steps move their bytes at 1 / 1.75 of the narrower ones' rate
+            gemm[1] *= 1.75
     elif v in (14, 18):
         mt, nt = -(-M // 256), -(-NO // 256)
         per = -(-(mt * nt) // XCDS)

@@ -2641,7 +2641,7 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
                             static_cast<int>(C), 0, 0, 0};
         return launch_wgrad(dtype, G, X, gw, gb, M, HD, C, workspace, ws_bytes, stream, &gp, stored);
     }
-    // the streaming GEMM (16-bit, C = 256, HD = 128 or 256, many tokens) reads W as stored too
+    // the streaming GEMM (16-bit, C = 256, HD = 128 or 256, or both 384, many tokens) reads W as stored too
     if (value_proj_plan(dtype, G, W, nullptr, gm, M, HD, C, 0, 0) == 22 && gemm_stream_fits(dtype, sp)) {
         rc = launch_gemm_stream(dtype, sp, stream, true);
         if (rc != 0) return rc;

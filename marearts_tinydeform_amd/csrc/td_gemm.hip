@@ -227,7 +227,7 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //   18 persistent 256 x 256 tiles fed by direct-to-LDS loads, one workgroup per CU (td_gemm_dma.hip; 16-bit,
 //      K % 64 == 0, gemm_persistent_fits)
 //   22 the streaming kernel: a quarter of W in each wavefront's registers, token rows streamed through LDS
-//      (td_gemm_stream.hip; 16-bit, NO = 256, K = 128 or 256)
+//      (td_gemm_stream.hip; 16-bit, NO = 256, K = 128 or 256, or NO = K = 384)
 //   23 64 x 32   4 waves of 16 x 32, one chunk of 256/128, one stage
 //   24 32 x 32   2 waves of 16 x 32, one chunk of 256/128, one stage
 //   25 64 x 64   4 waves of 16 x 64, K chunks of 128/64, two stages
@@ -237,7 +237,8 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //   256 outputs: the streaming kernel (22) from 14000 rows at K = 256 (M = 16384 8.3 µs against 9.1 for 25, M = 16800
 //     9.1 against 11.2 for 13 and 12.2 for 25, M = 33600 12.2 against 15.4, M = 67200 17.6 against 23.5; it loses at
 //     12000 rows, 7.8 against 7.4 for 25, and at 8400, 7.5 against 7.1), from 8000 rows at K = 128 (M = 8400 5.4
-//     against 5.6 for 25, M = 16384 6.1 against 7.0);
+//     against 5.6 for 25, M = 16384 6.1 against 7.0); 384 outputs of K = 384: from 10000 rows (M = 12000 11.3 against
+//     13.3 for 13, M = 84253 40.7 against 51.3; at 8400 10.8 for both);
 //   deep K (K >= 512, K % 64 == 0) on a grid of at least 200 tiles of 256 x 128, or more than one round (256) of
 //     128 x 128 tiles, or from 8000 rows: the direct-to-LDS kernels, persistent 256 x 256 tiles (18) from 120 of
 //     them, else 256 x 128 (14) (C = 1024: M = 43520 87-89 µs for 18 against 97-100 for the same tiles one per
@@ -271,7 +272,7 @@ int pick_variant(int dtype, const GemmParams& p) {
         if (p.K <= 256) return tiles_64 <= 40 ? 24 : tiles_64 <= 100 ? 23 : tiles_64 <= 1100 ? 25 : tiles_128 < 1024 ? 5 : 2;
         return tiles_64 < 512 ? 25 : 2;
     }
-    if (gemm_stream_fits(dtype, p) && p.M >= (p.K == 256 ? 14000 : 8000)) return 22;
+    if (gemm_stream_fits(dtype, p) && p.M >= (p.K == 256 ? 14000 : p.K == 384 ? 10000 : 8000)) return 22;
     const int64_t tiles_256x128 = ((p.M + 255) / 256) * static_cast<int64_t>((p.NO + 127) / 128);
     const int64_t tiles_256 = ((p.M + 255) / 256) * static_cast<int64_t>((p.NO + 255) / 256);
     if (p.K >= 512 && p.K % 64 == 0 && (tiles_256x128 >= 200 || tiles_128 > 256 || p.M >= 8000))

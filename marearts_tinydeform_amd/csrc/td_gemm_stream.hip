@@ -1,5 +1,6 @@
-// Streaming value projection for narrow K: value[M, 256] = memory[M, K] . W[256, K]^T + bias, K = 128 or 256,
-// 16-bit operands (the C = 256 projections of RT-DETR, DINO and Deformable-DETR decoders).
+// Streaming value projection for narrow K: value[M, 256] = memory[M, K] . W[256, K]^T + bias, K = 128 or 256, and
+// value[M, 384] at K = 384, 16-bit operands (the C = 256 projections of RT-DETR, DINO and Deformable-DETR decoders,
+// and twelve heads of 32).
 //
 // At K <= 256 the product is bound by HBM: each token row is read once (K * 2 bytes) and its value row written once
 // (512 bytes), 128 flops per byte, below MI355X's ridge. A tiled GEMM spends a tile's short life (K / 32 chunks)
@@ -31,12 +32,18 @@
 // staging W through LDS in whole lines, with the second stage requested at kernel start too: 16800 x 256
 // 9.0 -> 7.6, 33600 12.2 -> 10.3, 44446 14.0 -> 12.0, B8 bf16 17.8 -> 15.9, DINO B4 21.3 -> 18.8, 177784 33.7 ->
 // 32.8, 44446 x 128 9.9 -> 8.9. Stores that bypass or write through L2 (nontemporal, sc1) measured no faster.
+//
+// At K = 384 a wavefront's quarter of W is 96 channels, 288 of its 512 registers, and W (288 KB) passes through LDS 32
+// channels of each wavefront at a time. Bound by HBM and by moving part of W from accumulator registers (about 170 moves
+// a step of 144 MFMAs): 84253 x 384 x 384 bf16 51.3 us with the 128 x 128 LDS tiles, 45.4 with the direct-to-LDS ones,
+// 40.7 here (3.2 us a step, 3.9 TB/s); 30000 rows 19.6 -> 19.1, 16801 15.2 -> 14.5, 12000 13.3 -> 11.3.
 #include "td_gemm.h"
 
 namespace td {
 namespace {
 
-constexpr int kStreamNO = 256;   // output columns
+template <int NO>
+constexpr bool kWholeW = NO <= 256;  // W's LDS copy fits beside the token stages
 constexpr int kStreamWaves = 4;  // wavefronts per workgroup (one per SIMD)
 constexpr int kStreamStep = 32;  // tokens per step
 
@@ -73,16 +80,16 @@ __device__ __forceinline__ void meet() {
 // reads (ds_read_b64_tr_b16: within each 16 lanes, lane i receives element i % 4 of the 8-byte pieces lanes i / 4,
 // 4 + i / 4, 8 + i / 4 and 12 + i / 4 point at), lane j pointing at k row 8 kg + j / 4 (+ 4) and at the column of
 // its fragment layout's channel group j % 4, so that lane r receives the 8 k of the channel the layout gives it.
-template <typename T, int KB, bool WT>
+template <typename T, int KB, bool WT, int NO>
 __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_stream_kernel(
     GemmParams p) {
-    constexpr int NTQ = kStreamNO / 16 / kStreamWaves;  // 16-channel tiles per wavefront: 4
+    constexpr int NTQ = NO / 16 / kStreamWaves;         // 16-channel tiles per wavefront: 4 or 6
     constexpr int CHR = KB * 4;                         // 16-byte chunks per token row
     constexpr int ROWB = CHR * 16;                      // bytes per token row
     constexpr int STEP = kStreamStep;
     constexpr int SHN = STEP / 16;                      // 16-token halves per step
-    constexpr int STAGE = STEP * ROWB;                  // 16 KB (K = 256) or 8 KB (K = 128)
-    constexpr int DL = STAGE / 1024 / kStreamWaves;     // 1 KB direct loads per wavefront per stage: 4 or 2
+    constexpr int STAGE = STEP * ROWB;                  // 64 K bytes: 8 KB to 24 KB
+    constexpr int DL = STAGE / 1024 / kStreamWaves;     // 1 KB direct loads per wavefront per stage: 2 to 6
     constexpr int NST = SHN * (NTQ / 2);                // stores per wavefront per step
     static_assert(DL >= 1 && CHR >= 16 && CHR % 16 == 0, "stage layout");
     // Waits, in vector-memory operations that may stay in flight (they complete in issue order):
@@ -107,7 +114,7 @@ __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_pe
     if (ns <= 0) return;  // the whole workgroup (uniform)
     // the channel quarter of this wavefront, rotated by workgroup so that the CUs of an XCD request different parts
     // of W first
-    const int qc = 64 * ((wave + static_cast<int>(blockIdx.x / kXcds)) & 3);
+    const int qc = NO / kStreamWaves * ((wave + static_cast<int>(blockIdx.x / kXcds)) & 3);
 
     // direct loads of step i's token rows into stage i % 2; steps past the last re-read the last rows into a stage
     // that is never read, so every step issues the same loads and the waits stay exact
@@ -132,16 +139,15 @@ __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_pe
     u32x4 wf[NTQ][KB];
     unsigned char* const wl = smem + 2 * STAGE;  // the LDS copy of W
     auto wkey = [](int ch) { return (((ch >> 3) & 3) << 2) | (ch & 3); };
-    {
-        constexpr int WDL = kStreamNO * CHR / kWave / kStreamWaves;  // 1 KB direct loads per wavefront: CHR
+    if constexpr (kWholeW<NO>) {
+        constexpr int WDL = NO * CHR / kWave / kStreamWaves;  // 1 KB direct loads per wavefront: CHR
         const int rot = static_cast<int>(blockIdx.x / kXcds) % WDL;
 #pragma unroll 4
         for (int jj = 0; jj < WDL; ++jj) {
             const int j = wave * WDL + (jj + rot) % WDL;  // the CUs of an XCD start on different runs
             const int sl = j * kWave + lane;
             if constexpr (WT) {  // slot sl: k row sl / 32, channels (sl % 32) * 8 .. + 7
-                load_lds16(W + static_cast<size_t>(sl / (kStreamNO / 8)) * kStreamNO + (sl % (kStreamNO / 8)) * 8,
-                           wl + j * 1024);
+                load_lds16(W + static_cast<size_t>(sl / (NO / 8)) * NO + (sl % (NO / 8)) * 8, wl + j * 1024);
             } else {
                 const int ch = sl / CHR, c = (sl % CHR) ^ wkey(ch);
                 load_lds16(W + static_cast<size_t>(ch) * K + c * 8, wl + j * 1024);
@@ -200,25 +206,72 @@ __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_pe
     // left for the compiler to wait on (with step 0 inside, its merged count put a full wait after every step's
     // direct loads). A stage is refilled only after every wavefront has passed the barrier of the step that follows
     // its reads.
-    meet<0>();  // stages 0 and 1, W and the bias have landed
+    using v4s = short __attribute__((ext_vector_type(4)));
+    using lds_v4s = __attribute__((address_space(3))) v4s;
+    if constexpr (kWholeW<NO>) {
+        meet<0>();  // stages 0 and 1, W and the bias have landed
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-        for (int t = 0; t < NTQ; ++t) {
-            if constexpr (WT) {
-                using v4s = short __attribute__((ext_vector_type(4)));
-                using lds_v4s = __attribute__((address_space(3))) v4s;
-                const int k = kb * 32 + kg * 8 + (r >> 2);
-                const int col = qc + 32 * (t >> 1) + 8 * (r & 3) + 4 * (t & 1);
-                const unsigned char* q = wl + (k * kStreamNO + col) * 2;
-                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q));
-                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q + 4 * kStreamNO * 2));
-                wf[t][kb] = __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            } else {
-                const int ch = qc + 32 * (t >> 1) + 8 * (r >> 2) + 4 * (t & 1) + (r & 3);
-                wf[t][kb] = *reinterpret_cast<const u32x4*>(wl + (ch * CHR + ((kb * 4 + kg) ^ wkey(ch))) * 16);
+            for (int t = 0; t < NTQ; ++t) {
+                if constexpr (WT) {
+                    const int k = kb * 32 + kg * 8 + (r >> 2);
+                    const int col = qc + 32 * (t >> 1) + 8 * (r & 3) + 4 * (t & 1);
+                    const unsigned char* q = wl + (k * NO + col) * 2;
+                    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q));
+                    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q + 4 * NO * 2));
+                    wf[t][kb] = __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                } else {
+                    const int ch = qc + 32 * (t >> 1) + 8 * (r >> 2) + 4 * (t & 1) + (r & 3);
+                    wf[t][kb] = *reinterpret_cast<const u32x4*>(wl + (ch * CHR + ((kb * 4 + kg) ^ wkey(ch))) * 16);
+                }
             }
+    } else {
+        // W does not fit beside the stages: 32 of this wavefront's channels at a time, through LDS of its own (rows of
+        // K, or with WT the K rows of those channels), so that no barrier is needed
+        unsigned char* const own = wl + wave * (32 * ROWB);
+#pragma unroll
+        for (int pp = 0; pp < NTQ / 2; ++pp) {
+            constexpr int WDL = 32 * ROWB / 1024;
+#pragma unroll 4
+            for (int j = 0; j < WDL; ++j) {
+                const int sl = j * kWave + lane;
+                if constexpr (WT) {  // slot sl: k row sl / 4, channels (sl % 4) * 8 .. + 7
+                    load_lds16(W + static_cast<size_t>(sl >> 2) * NO + qc + 32 * pp + (sl & 3) * 8, own + j * 1024);
+                } else {
+                    const int ch = sl / CHR, c = (sl % CHR) ^ wkey(ch);
+                    load_lds16(W + static_cast<size_t>(qc + 32 * pp + ch) * K + c * 8, own + j * 1024);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): they have landed
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if constexpr (WT) {
+                        const unsigned char* q = own + ((kb * 32 + kg * 8 + (r >> 2)) * 32 + 8 * (r & 3) + 4 * h) * 2;
+                        const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q));
+                        const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(q + 4 * 32 * 2));
+                        wf[2 * pp + h][kb] =
+                            __builtin_bit_cast(u32x4, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                    } else {
+                        const int ch = 8 * (r >> 2) + 4 * h + (r & 3);
+                        wf[2 * pp + h][kb] =
+                            *reinterpret_cast<const u32x4*>(own + (ch * CHR + ((kb * 4 + kg) ^ wkey(ch))) * 16);
+                    }
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0): they are read
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
         }
+        meet<0>();  // stages 0 and 1 and the bias have landed
+    }
     step(0);
     for (int i = 1; i < ns; ++i) {
         meet<VM_STEADY>();
@@ -230,19 +283,20 @@ __global__ __launch_bounds__(kStreamWaves* kWave) __attribute__((amdgpu_waves_pe
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
 }
 
-template <typename T, int KB, bool WT>
+template <typename T, int KB, bool WT, int NO>
 int go_stream(GemmParams p, int64_t grid, hipStream_t stream) {
-    // two token stages and W: 160 KB at K = 256, 80 KB at K = 128
-    constexpr size_t lds = static_cast<size_t>(2) * kStreamStep * KB * 64 + static_cast<size_t>(kStreamNO) * KB * 64;
+    // two token stages and W: 160 KB at K = 256, 80 KB at K = 128; 144 KB at K = 384
+    constexpr size_t lds =
+        static_cast<size_t>(2) * kStreamStep * KB * 64 + static_cast<size_t>(kWholeW<NO> ? NO : 32 * kStreamWaves) * KB * 64;
     if constexpr (lds > 65536) {
         static std::atomic<uint64_t> done{0};
-        const hipError_t attr =
-            allow_dynamic_lds(reinterpret_cast<const void*>(gemm_stream_kernel<T, KB, WT>), static_cast<int>(lds), done);
+        const hipError_t attr = allow_dynamic_lds(reinterpret_cast<const void*>(gemm_stream_kernel<T, KB, WT, NO>),
+                                                  static_cast<int>(lds), done);
         if (attr != hipSuccess)
             return set_error(-3, "value_proj: LDS size attribute refused: %s", hipGetErrorString(attr));
     }
-    hipLaunchKernelGGL((gemm_stream_kernel<T, KB, WT>), dim3(static_cast<unsigned>(grid)), dim3(kStreamWaves * kWave), lds,
-                       stream, p);
+    hipLaunchKernelGGL((gemm_stream_kernel<T, KB, WT, NO>), dim3(static_cast<unsigned>(grid)), dim3(kStreamWaves * kWave),
+                       lds, stream, p);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? 0 : set_error(-3, "value_proj launch failed: %s", hipGetErrorString(e));
 }
@@ -254,7 +308,8 @@ int stream_t(GemmParams p, hipStream_t stream) {
     const int cus = cu_count();
     if (grid > cus) grid = cus;
     if (grid < 1) grid = 1;
-    return p.K == 256 ? go_stream<T, 8, WT>(p, grid, stream) : go_stream<T, 4, WT>(p, grid, stream);
+    if (p.NO == 384) return go_stream<T, 12, WT, 384>(p, grid, stream);
+    return p.K == 256 ? go_stream<T, 8, WT, 256>(p, grid, stream) : go_stream<T, 4, WT, 256>(p, grid, stream);
 }
 
 }  // namespace
@@ -263,8 +318,9 @@ int stream_t(GemmParams p, hipStream_t stream) {
 bool gemm_stream_fits(int dtype, const GemmParams& p) {
     const uintptr_t al = reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.w) |
                          reinterpret_cast<uintptr_t>(p.c) | reinterpret_cast<uintptr_t>(p.bias);
-    return (dtype == kF16 || dtype == kBF16) && p.NO == kStreamNO && (p.K == 128 || p.K == 256) && p.M > 0 &&
-           al % 16 == 0 && p.hm_D % 8 == 0;
+    return (dtype == kF16 || dtype == kBF16) &&
+           ((p.NO == 256 && (p.K == 128 || p.K == 256)) || (p.NO == 384 && p.K == 384)) && p.M > 0 && al % 16 == 0 &&
+           p.hm_D % 8 == 0;
 }
 
 int launch_gemm_stream(int dtype, GemmParams p, hipStream_t stream, bool w_stored) {
