@@ -15,10 +15,11 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (4, 8, 32, 4, [(55, 57), (28, 29), (14, 15)]),
     (2, 8, 64, 8, [(65, 67), (61, 66)]),
-    (1, 2, 32, 4, [(33, 49), (17, 25), (9, 13), (5, 7), (3, 4)]),
-    (1, 2, 64, 4, [(31, 47), (16, 24)]),
-    (2, 2, 16, 16, [(24, 39)]),
-    (1, 4, 8, 2, [(9, 5), (40, 3)]),
+    (4, 4, 32, 4, [(33, 49), (17, 25), (9, 13), (5, 7), (3, 4)]),
+    (8, 3, 64, 4, [(31, 47), (16, 24)]),
+    (6, 6, 16, 16, [(24, 39)]),
+    (8, 8, 8, 2, [(25, 15), (40, 5)]),
+    (1, 2, 32, 4, [(31, 47), (16, 24)]),    # under 32768 rows: consecutive queries
 ]
 
 
@@ -44,26 +45,28 @@ def test_tile_scatter(shape, dtype):
 
 def test_tile_scatter_keeps_infinities_where_they_belong():
     # an infinite grad_out row reaches the pixels it samples and no other, in float16 too
-    levels = [(20, 30), (10, 15)]
+    levels = [(80, 100), (40, 50)]
     N = sum(h * w for h, w in levels)
-    args = workload(1, N, 2, 32, 64, levels, 4, torch.float16, loc_dist='encoder', seed=2)
+    args = workload(1, N, 4, 32, 128, levels, 4, torch.float16, loc_dist='encoder', seed=2)
     # corners of non-zero weight only (0 times infinity is NaN, here as anywhere)
-    args[5][0, 100] = torch.linspace(0.2131, 0.4377, 2 * 2 * 4 * 2).view(2, 2, 4, 2).half()
+    args[5][0, 100] = torch.linspace(0.2131, 0.4377, 4 * 2 * 4 * 2).view(4, 2, 4, 2).half()
     for l, (h, w) in enumerate(levels):
         pix = args[5][0, 100, :, l].float() * torch.tensor([w, h]) - 0.5
+        args[5][0, 100, :, l] += (pix == pix.floor()).half() * 0.001    # off the pixel centres
+        pix = args[5][0, 100, :, l].float() * torch.tensor([w, h]) - 0.5
         assert (pix != pix.floor()).all()
-    value = torch.randn(1, N, 64, generator=torch.Generator().manual_seed(1)).half()
-    go = torch.ones(1, N, 64).half()
+    value = torch.randn(1, N, 128, generator=torch.Generator().manual_seed(1)).half()
+    go = torch.ones(1, N, 128).half()
     go[0, 100, :32] = float('inf')          # head 0 of query 100
     dev = [t.cuda() for t in (value, args[3], args[4], args[5], args[6])]
-    gv, _, _ = _native.sample_backward(dev[0], 2, dev[1], dev[2], dev[3], dev[4], go.cuda())
+    gv, _, _ = _native.sample_backward(dev[0], 4, dev[1], dev[2], dev[3], dev[4], go.cuda())
     bad = (~gv.isfinite()).any(-1)[0].cpu()
     assert torch.isfinite(gv[0, :, 32:]).all()
     go[0, 100, :32] = 0
     go[0, :100] = 0
     go[0, 101:] = 0
     go[0, 100, :32] = 1
-    alone, _, _ = _native.sample_backward(dev[0], 2, dev[1], dev[2], dev[3], dev[4], go.cuda())
+    alone, _, _ = _native.sample_backward(dev[0], 4, dev[1], dev[2], dev[3], dev[4], go.cuda())
     hit = (alone[0, :, :32] != 0).any(-1).cpu()
     assert hit.any() and bool((bad == hit).all())
 
