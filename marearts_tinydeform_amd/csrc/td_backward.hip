@@ -1400,13 +1400,16 @@ struct SortParams {
     FastDiv d_lp;
 };
 
-// The bins of the levels: level l's tokens start[l] .. start[l] + n[l] - 1 (clamped into [0, N)) in bins of
-// 2^shift[l] tokens, numbered base[l] .. base[l + 1] - 1 (base[L] = the bins in use, at most sp.nb).
+// The bins of the levels: level l's tokens start[l] .. start[l] + n[l] - 1 (those in [0, N)) in bins of
+// 2^shift[l] tokens, numbered from base[l]; `bins` in all, at most sp.nb. Every token is in exactly one bin, which
+// writes its sum: where the levels do not hold each token of [0, N) exactly once (tokens of no level, or shared by
+// levels), every level stands for the whole range, in the same bins of 2^min_shift tokens.
 struct SortLevels {
-    int base[kMaxLevelPoints + 1];
+    int base[kMaxLevelPoints];
     int shift[kMaxLevelPoints];
     int start[kMaxLevelPoints];
     int n[kMaxLevelPoints];
+    int bins;
 };
 
 // A reduce item: bin tokens t0 .. t0 + 2^shift - 1 of (b, h) = bh, of which `tokens` exist, range k of 2^j of them;
@@ -1437,23 +1440,39 @@ __device__ inline SortItem sort_item_unpack(const uint4& u) {
 __device__ void sort_levels(const SortParams& sp, SortLevels& lv) {
     const Geom& g = sp.g;
     const int l = lane_id();
-    int nbins = 0;
+    int s0 = 0, n = 0, nbins = 0;  // lane l's level: first token and tokens
+    int64_t corners = 0;
     if (l < g.L) {
         const int64_t st = g.starts[l], n64 = g.shapes[2 * l] * g.shapes[2 * l + 1];
-        const int64_t s0 = st < 0 ? 0 : (st > g.N ? g.N : st);
-        const int64_t n = n64 < 0 ? 0 : (n64 > g.N - s0 ? g.N - s0 : n64);
+        const int64_t lo = min(max(st, int64_t{0}), static_cast<int64_t>(g.N));
+        s0 = static_cast<int>(lo);
+        n = static_cast<int>(min(max(st + n64, lo), static_cast<int64_t>(g.N)) - lo);
         const int pl = g.P > 0 ? g.P : g.level_end[l] - (l > 0 ? g.level_end[l - 1] : 0);
-        const int64_t corners = int64_t{4} * g.Q * pl;
+        corners = int64_t{4} * g.Q * pl;
+    }
+    // each token once: the levels end to end and N tokens in all, or in any other order without an overlap
+    const int upto = wave_incl_scan(n);
+    bool one = __builtin_amdgcn_readlane(upto, kWave - 1) != g.N;
+    if (!one && __any(n > 0 && s0 != upto - n)) {  // uniform
+        bool shared = false;
+        for (int j = 0; j < g.L; ++j) {
+            const int sj = __builtin_amdgcn_readlane(s0, j), nj = __builtin_amdgcn_readlane(n, j);
+            if (j != l && n > 0 && nj > 0) shared |= s0 < sj + nj && sj < s0 + n;
+        }
+        one = __any(shared);
+    }
+    if (one) s0 = 0, n = g.N;
+    if (l < g.L) {
         int shift = sp.min_shift;
-        while (shift < sp.tb_shift && (corners << (shift + 1)) <= int64_t{kSortTarget} * n) ++shift;
-        nbins = static_cast<int>((n + (int64_t{1} << shift) - 1) >> shift);
+        while (!one && shift < sp.tb_shift && (corners << (shift + 1)) <= int64_t{kSortTarget} * n) ++shift;
+        nbins = (n + (1 << shift) - 1) >> shift;
         lv.shift[l] = shift;
-        lv.start[l] = static_cast<int>(s0);
-        lv.n[l] = static_cast<int>(n);
+        lv.start[l] = s0;
+        lv.n[l] = n;
     }
     const int incl = wave_incl_scan(nbins);
-    if (l < g.L) lv.base[l + 1] = min(incl, sp.nb);
-    if (l == 0) lv.base[0] = 0;
+    if (l < g.L) lv.base[l] = one ? 0 : incl - nbins;
+    if (l == g.L - 1) lv.bins = one ? nbins : incl;
 }
 
 // Thread tid of tile (bh, qt): its sample's four corners (tokens, -1 outside) and coefficients, its level and row.
@@ -1488,13 +1507,12 @@ __device__ __forceinline__ bool sort_sample(const SortParams& sp, int bh, int qt
     return true;
 }
 
-// The bin of token tk of level l and its position in the bin (-1 for a token outside the level's clamped range)
+// The bin of token tk of level l and its position in the bin (-1 for a token outside the level's range)
 __device__ __forceinline__ int sort_bin_of(const SortLevels& lv, int l, int tk, int& pos) {
     const int rel = tk - lv.start[l];
     if (static_cast<unsigned>(rel) >= static_cast<unsigned>(lv.n[l])) return -1;
-    const int bin = lv.base[l] + (rel >> lv.shift[l]);
     pos = rel & ((1 << lv.shift[l]) - 1);
-    return bin < lv.base[l + 1] ? bin : -1;
+    return lv.base[l] + (rel >> lv.shift[l]);
 }
 
 template <typename T>
@@ -1509,7 +1527,7 @@ __global__ __launch_bounds__(256) void sort_count_kernel(SortParams sp) {
     const bool has = sort_sample<T>(sp, bh, qt, threadIdx.x, tk, cf, lev, row);  // its loads overlap the table's
     if (threadIdx.x < kWave) sort_levels(sp, lv);
     __syncthreads();  // the level table and the cleared counters
-    const int nb = lv.base[sp.g.L];
+    const int nb = lv.bins;
     if (has) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -1559,7 +1577,7 @@ __device__ __forceinline__ void sort_scan_body(const SortParams& sp, int bh, uns
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & (kWave - 1);
     if (tid < kWave) sort_levels(sp, lv);
     __syncthreads();
-    const int nb = lv.base[sp.g.L];
+    const int nb = lv.bins;
     int* hist = sp.hist + static_cast<int64_t>(bh) * sp.nb * sp.qtiles;
     const int n = nb * sp.qtiles;  // < 2^30 (checked on the host)
     int* mine = v + tid * (kScanK + 1);
