@@ -759,6 +759,30 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
     return v + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
+// Level l's tokens in [0, N): the first and how many
+struct LevelTokens {
+    int first, n;
+};
+__device__ __forceinline__ LevelTokens level_tokens(const Geom& g, int64_t st, int64_t size) {
+    const int64_t lo = min(max(st, int64_t{0}), static_cast<int64_t>(g.N));
+    return {static_cast<int>(lo), static_cast<int>(min(max(st + size, lo), static_cast<int64_t>(g.N)) - lo)};
+}
+
+// Whether each token of [0, N) lies in exactly one level: the levels end to end, or in another order N tokens in all
+// without an overlap. Lane l holds level l's tokens (n = 0: no such level); a whole wavefront, every lane active.
+__device__ __forceinline__ bool levels_hold_once(const Geom& g, LevelTokens t) {
+    const int end = t.first + t.n, l = lane_id();
+    const int before = __builtin_amdgcn_update_dpp(0, end, 0x138, 0xf, 0xf, false);  // wave_shr:1; lane 0: 0
+    if (__builtin_amdgcn_readlane(end, g.L - 1) == g.N && !__any(l < g.L && t.first != before)) return true;
+    if (__builtin_amdgcn_readlane(wave_incl_scan(t.n), kWave - 1) != g.N) return false;
+    bool shared = false;
+    for (int j = 0; j < g.L; ++j) {
+        const int sj = __builtin_amdgcn_readlane(t.first, j), nj = __builtin_amdgcn_readlane(t.n, j);
+        if (j != l && t.n > 0 && nj > 0) shared |= t.first < sj + nj && sj < t.first + t.n;
+    }
+    return !__any(shared);
+}
+
 template <typename T, int NTH>
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void scatter_bucket_kernel(BucketParams bp) {
     using A = float;
@@ -975,8 +999,8 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void s
     tile(bh / g.H, bh % g.H, [&](int r) { return r < nq ? q0 + r : -1; });
 }
 
-// The same scatter for self-attention (Q = N, query q at token q's pixel), a workgroup a tile of 16 x 16 or 16 x 8
-// pixels of a level's map: those queries of one head touch 10.2 and 7.9 times fewer pixels than they have corners on
+// The same scatter for self-attention (Q = N; where the levels tile the tokens, query q lies at token q's pixel), a
+// workgroup a tile of 16 x 16 or 16 x 8 pixels of a level's map: those queries of one head touch 10.2 and 7.9 times fewer pixels than they have corners on
 // DINO-style inputs (8 x 4 pixels: 4.3), and the float atomics, one D-wide line a touched pixel, run at 320 G lanes/s
 // whatever else is done (200 and 260 us at the DINO encoder). So the rest has to run beside them: the barriers wait for
 // LDS only, nothing inside a tile waits for a load, and a level costs three barriers:
@@ -1077,7 +1101,11 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
         nbx = (width(l) + tp.tw - 1) >> tp.tw_shift;
         return nbx * ((height(l) + tp.th - 1) >> tp.th_shift);
     };
-    int per_bh = 0;
+    // Every query is visited once wherever the levels lie: one whose token several levels hold, in the first of them;
+    // those of no level, in tiles of a further map tw pixels wide of all the tokens
+    const bool once = levels_hold_once(
+        g, lane < g.L ? level_tokens(g, level_st, static_cast<int64_t>(level_w) * level_h) : LevelTokens{0, 0});
+    int per_bh = once ? 0 : (g.N + QT - 1) >> (tp.tw_shift + tp.th_shift);
     for (int l = 0; l < g.L; ++l) {
         int nbx;
         per_bh += level_tiles(l, nbx);
@@ -1092,16 +1120,31 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
             if (rest < n) break;
             rest -= n;
         }
-        const int wq = width(lq), hq = height(lq);
+        const bool further = lq == g.L;
+        const int wq = further ? tp.tw : width(lq), hq = further ? (g.N + tp.tw - 1) >> tp.tw_shift : height(lq);
+        const int64_t stq = further ? 0 : start(lq);
+        if (further) nbx = 1;
         const int qx = (rest % nbx) * tp.tw, qy = (rest / nbx) * tp.th;
         const int nx = min(tp.tw, wq - qx), ny = min(tp.th, hq - qy);
-        const int64_t stq = start(lq);
-        // the query of row r; -1: none (past the map, or a token that is not in [0, N))
-        auto query_of = [&](int r) {
+        // the token of row r; -1: none (past the map, or not in [0, N))
+        auto token_of = [&](int r) {
             const int y = r >> tp.tw_shift, x = r & (tp.tw - 1);
             const int64_t q = stq + static_cast<int64_t>(qy + y) * wq + qx + x;
             return x < nx && y < ny && q >= 0 && q < g.Q ? static_cast<int>(q) : -1;
         };
+        // its query; -1 also where another tile visits it. By a whole wavefront: it reads the levels' lanes
+        auto query_of = [&](int r) {
+            int q = token_of(r);
+            if (!once)
+                for (int l = 0; l < lq; ++l)
+                    if (q >= start(l) && q < start(l) + static_cast<int64_t>(width(l)) * height(l)) q = -1;
+            return q;
+        };
+        if (!once) {  // a tile without a query, which every wavefront sees for itself
+            bool any = false;
+            for (int r0 = 0; r0 < QT; r0 += kWave) any |= query_of(min(r0 + lane, QT - 1)) >= 0;
+            if (!__any(any)) continue;
+        }
         A* __restrict__ gv =
             static_cast<A*>(tp.grad_value) + static_cast<int64_t>(b) * g.N * HD + static_cast<int64_t>(h) * D;
 
@@ -1128,7 +1171,7 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
 
         // this thread's samples: point jp of row r, level by level
         const int r = static_cast<int>(fast_div(tp.d_p, static_cast<uint32_t>(tid))), jp = tid - r * P;
-        const int q = r < QT ? query_of(r) : -1;
+        const int qr = query_of(min(r, QT - 1)), q = r < QT ? qr : -1;
         const int64_t first = ((static_cast<int64_t>(b) * g.Q + (q >= 0 ? q : 0)) * g.H + h) * g.LP + jp;
         // the samples of kAhead levels, loaded and waited for before any of their atomics: a wavefront's vector memory
         // operations complete in order, and a wait inside the levels' loop would be one for the atomics
@@ -1153,7 +1196,7 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
         load(0);
         meet_lds();  // every wavefront is done with the previous tile's rows
         for (int i = tid; i < QT * D; i += kTileThreads) {
-            const int row = i >> tp.d_shift, qr = query_of(row);
+            const int row = i >> tp.d_shift, qr = token_of(row);
             s.gr[i] = qr >= 0 ? go[(static_cast<int64_t>(b) * g.Q + qr) * HD + static_cast<int64_t>(h) * D + (i - row * D)]
                               : T(0);
         }
@@ -1440,35 +1483,23 @@ __device__ inline SortItem sort_item_unpack(const uint4& u) {
 __device__ void sort_levels(const SortParams& sp, SortLevels& lv) {
     const Geom& g = sp.g;
     const int l = lane_id();
-    int s0 = 0, n = 0, nbins = 0;  // lane l's level: first token and tokens
+    LevelTokens t{0, 0};  // lane l's level's
+    int nbins = 0;
     int64_t corners = 0;
     if (l < g.L) {
-        const int64_t st = g.starts[l], n64 = g.shapes[2 * l] * g.shapes[2 * l + 1];
-        const int64_t lo = min(max(st, int64_t{0}), static_cast<int64_t>(g.N));
-        s0 = static_cast<int>(lo);
-        n = static_cast<int>(min(max(st + n64, lo), static_cast<int64_t>(g.N)) - lo);
+        t = level_tokens(g, g.starts[l], g.shapes[2 * l] * g.shapes[2 * l + 1]);
         const int pl = g.P > 0 ? g.P : g.level_end[l] - (l > 0 ? g.level_end[l - 1] : 0);
         corners = int64_t{4} * g.Q * pl;
     }
-    // each token once: the levels end to end and N tokens in all, or in any other order without an overlap
-    const int upto = wave_incl_scan(n);
-    bool one = __builtin_amdgcn_readlane(upto, kWave - 1) != g.N;
-    if (!one && __any(n > 0 && s0 != upto - n)) {  // uniform
-        bool shared = false;
-        for (int j = 0; j < g.L; ++j) {
-            const int sj = __builtin_amdgcn_readlane(s0, j), nj = __builtin_amdgcn_readlane(n, j);
-            if (j != l && n > 0 && nj > 0) shared |= s0 < sj + nj && sj < s0 + n;
-        }
-        one = __any(shared);
-    }
-    if (one) s0 = 0, n = g.N;
+    const bool one = !levels_hold_once(g, t);
+    if (one) t = LevelTokens{0, g.N};
     if (l < g.L) {
         int shift = sp.min_shift;
-        while (!one && shift < sp.tb_shift && (corners << (shift + 1)) <= int64_t{kSortTarget} * n) ++shift;
-        nbins = (n + (1 << shift) - 1) >> shift;
+        while (!one && shift < sp.tb_shift && (corners << (shift + 1)) <= int64_t{kSortTarget} * t.n) ++shift;
+        nbins = (t.n + (1 << shift) - 1) >> shift;
         lv.shift[l] = shift;
-        lv.start[l] = s0;
-        lv.n[l] = n;
+        lv.start[l] = t.first;
+        lv.n[l] = t.n;
     }
     const int incl = wave_incl_scan(nbins);
     if (l < g.L) lv.base[l] = one ? 0 : incl - nbins;

@@ -72,3 +72,17 @@ def test_decoder_gradients(kind, dtype):
     # 2^18 corners and more: the binned value gradient. A hot spot makes split bins
     compare(kind, 2, 350, 8, 32, [(40, 60), (20, 30), (10, 15)], 4, dtype, 'uniform')
     compare(kind, 2, 350, 8, 16, [(40, 60), (20, 30), (10, 15)], 4, dtype, 'clustered', masked=True)
+
+
+@pytest.mark.parametrize('kind', KINDS)
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+def test_self_attention_gradients(kind, dtype):
+    # as many queries as tokens, 32768 rows and more: a query counts once whether its token lies in no level, one or two
+    compare(kind, 6, None, 4, 64, [(33, 49), (21, 35)], 4, dtype, 'encoder')
+    compare(kind, 7, None, 5, 32, [(29, 40), (24, 31)], 4, dtype, 'encoder', masked=True)
+
+
+def test_self_attention_gradients_large_tiles():
+    # the 16-bit form from 131072 rows
+    for kind in ('gaps', 'shared', 'same'):
+        compare(kind, 4, None, 8, 32, [(55, 85), (28, 36), (14, 15)], 4, torch.bfloat16, 'encoder', masked=kind == 'gaps')
