@@ -2112,10 +2112,11 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradParams p, int per_xcd) 
 // The weight gradient of float32 operands on the bfloat16 matrix units (td_split.h): the same tiles, splits and partials,
 // in steps of 32 tokens. Each thread takes 4 tokens x 4 columns of each operand, turns and splits them in registers,
 // and stores 8 bytes (4 tokens) a column and part; the next step's are loaded during the MFMAs, and two workgroups
-// share a CU, so that one splits while the other's MFMAs run. A step with values beyond the split is added by float32
-// FMAs. Against the float32 units (us, with the reduce): 67200 x 256 x 256 123.8 -> 80.5, 16800 47.1 -> 36.0, 20000 x
-// 512 x 512 138.5 -> 86.1, 21760 x 1024 x 1024 501.8 -> 301.5 (0.91 PFLOP/s of bfloat16 products; what is left beside
-// the MFMAs are a step's split, its two barriers and the loads behind them).
+// share a CU, so that one splits while the other's MFMAs run. A step with values beyond the split's range (SplitRange) is
+// added on the float32 units, from memory (67200 x 256 x 256 with such a value in every step: 155 us). Against the
+// float32 units (us, with the reduce): 67200 x 256 x 256 123.8 -> 80.5, 16800 47.1 -> 36.0, 20000 x 512 x 512 138.5 ->
+// 86.1, 21760 x 1024 x 1024 501.8 -> 301.5 (0.91 PFLOP/s of bfloat16 products; what is left beside the MFMAs are a
+// step's split, its two barriers and the loads behind them).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void wgrad_split_kernel(WgradParams p,
                                                                                                   int per_xcd) {
     __shared__ __align__(16) SplitSlices s;
@@ -2142,14 +2143,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             px[u] = m < m_end && xcol ? *reinterpret_cast<const f32x4*>(X + static_cast<int64_t>(m) * p.K + c0 + cb) : zero;
         }
     };
-    bool beyond = false;
+    SplitRange range;
     auto stage = [&](const f32x4 (&v)[4], bf16* to) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const f32x4 col = {v[0][e], v[1][e], v[2][e], v[3][e]};
             bf16x4 part[3];
             split3(col, part[0], part[1], part[2]);
-            beyond |= beyond_split(col);
+            range.add(col);
             bf16* const at = to + split_at(cb + e, tq >> 1) + (tq & 1) * 4;
 #pragma unroll
             for (int o = 0; o < 3; ++o) *reinterpret_cast<bf16x4*>(at + o * kSplitPlane) = part[o];
@@ -2162,28 +2163,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int j = 0; j < 4; ++j) acc[i][j] = zero;
     load(m_begin);
     for (int m0 = m_begin; m0 < m_end; m0 += 32) {
-        beyond = false;
+        range = SplitRange();
         stage(pg, s.a);
         stage(px, s.b);
         if (do_b) bsum += (pg[0] + pg[1]) + (pg[2] + pg[3]);
-        const bool any = __any(beyond);
+        const bool any = __any(range.beyond());
         if (lane == 0) s.flags[wave] = any;
         __syncthreads();
         if (m0 + 32 < m_end) load(m0 + 32);  // in flight during this step's MFMAs
-        if (s.flags[0] | s.flags[1] | s.flags[2] | s.flags[3]) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int n = n0 + 64 * wa + 16 * i + 4 * kg + e, c = c0 + 64 * wb + 16 * j + r;
-                        if (n >= p.NO || c >= p.K) continue;
+        if (s.flags[0] | s.flags[1] | s.flags[2] | s.flags[3]) {  // on the float32 units, from memory
 #pragma unroll 1
-                        for (int m = m0; m < min(m0 + 32, m_end); ++m)
-                            acc[i][j][e] = fmaf(G[static_cast<int64_t>(m) * p.NO + n],
-                                                X[static_cast<int64_t>(m) * p.K + c], acc[i][j][e]);
-                    }
+            for (int k = 0; k < 32; k += 4) {
+                const int m = m0 + k + kg;
+                float a[4], b[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int n = n0 + 64 * wa + 16 * i + r, c = c0 + 64 * wb + 16 * i + r;
+                    a[i] = m < m_end && n < p.NO ? G[static_cast<int64_t>(m) * p.NO + n] : 0.f;
+                    b[i] = m < m_end && c < p.K ? X[static_cast<int64_t>(m) * p.K + c] : 0.f;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+            }
         } else {
             split_mma(s, wa, wb, lane, acc);
         }

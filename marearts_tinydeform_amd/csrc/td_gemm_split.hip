@@ -10,6 +10,9 @@
 //     the split's VALU work (about 900 cycles a step) runs beside the other's MFMAs (6144 for the two).
 //   * The product is formed transposed, D = W . tokens^T, and the rows of the output tiles are permuted, so that a
 //     lane ends with 8 consecutive channels of a token (two 16-byte stores; 128 bytes by the lanes of a token).
+//   * A step with a value beyond the split's range (SplitRange), or every step where W has one, runs on the float32
+//     units, its operands straight from memory: 67200 x 256 x 256 161 us with an infinite weight, against 97 on the
+//     register tiles (by scalar FMAs it was 8200).
 //   * A plane's row is K / 8 chunks of 16 bytes, chunk c at slot c ^ (row & 15), which an LDS probe reads at the full
 //     rate (525 B/ns a CU; unpermuted or padded by 16 bytes: 290).
 // Bound by the MFMAs: 67200 x 256 x 256 (52.8 GFLOP in six products) 55-60 us against 100 on the float32 units, of
@@ -70,7 +73,7 @@ template <int KB, bool WT>
 __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_split_kernel(
     GemmParams p) {
     constexpr int K = KB * 32;
-    constexpr int STEP = kSplitStep;
+    constexpr int STEP = kSplitStep;                          // two halves of 16 tokens
     constexpr int RAW_ROW = K * 4, ROWB = K * 2;              // bytes of a token row: float32, one plane
     constexpr int PLANE = STEP * ROWB, BUF = 3 * PLANE;
     constexpr int TOK = STEP / kSplitWaves;                   // tokens a wavefront loads and splits: 4
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
     auto split = [&](int i) {
         unsigned char* const dst = planes + (i & 1) * BUF;
         const int ln = unhoisted(lane);
-        bool beyond = false;
+        SplitRange range;
 #pragma unroll
         for (int j = 0; j < DL; ++j) {
             const int q = j * kWave + ln;
@@ -118,13 +121,13 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
             const int row = wave * TOK + q / (RAW_ROW / 16), c = q % (RAW_ROW / 16);
             bf16x4 h, m, l;
             split3(x, h, m, l);
-            beyond |= beyond_split(x);
+            range.add(x);
             unsigned char* const at = dst + row * ROWB + ((((c >> 1) ^ (row & 15)) << 4) | ((c & 1) << 3));
             *reinterpret_cast<bf16x4*>(at) = h;
             *reinterpret_cast<bf16x4*>(at + PLANE) = m;
             *reinterpret_cast<bf16x4*>(at + 2 * PLANE) = l;
         }
-        const bool any = __any(beyond);
+        const bool any = __any(range.beyond());
         if (lane == 0) flags[(i & 1) * kSplitWaves + wave] = any;
     };
 
@@ -137,7 +140,7 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
     {
         constexpr int WDL = 16 * RAW_ROW / 1024;                       // direct loads: 16 (K = 256) or 8
         unsigned char* const wl = smem + wave * (16 * RAW_ROW);
-        bool beyond = false;
+        SplitRange range;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             // tile t's row j is channel c0 + 8 (j / 4) + 4 t + j % 4
@@ -166,7 +169,8 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
                     for (int e = 0; e < 2; ++e)
                         x[e] = *reinterpret_cast<const f32x4*>(wl + r * RAW_ROW + (((k / 4 + e) ^ r) << 4));
                 }
-                beyond |= beyond_split(x[0]) | beyond_split(x[1]);
+                range.add(x[0]);
+                range.add(x[1]);
                 bf16x4 part[2][3];
 #pragma unroll
                 for (int e = 0; e < 2; ++e) split3(x[e], part[e][0], part[e][1], part[e][2]);
@@ -177,7 +181,7 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
             }
             wait_lds();
         }
-        const bool any = __any(beyond);
+        const bool any = __any(range.beyond());
         if (lane == 0) flags[2 * kSplitWaves + wave] = any;
     }
     if (tid < kSplitNO) bias_l[tid] = bias_v;
@@ -197,17 +201,52 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
 
     auto product = [&](int i) {
         const int rows = min(hi - (lo + STEP * i), STEP);
-        if (w_beyond || flagged(i & 1)) {  // every row of this step by float32 FMAs, in order of k
-#pragma unroll 1
-            for (int e = unhoisted(tid); e < rows * kSplitNO; e += kSplitWaves * kWave) {
-                const int m = lo + STEP * i + e / kSplitNO, n = e % kSplitNO;
-                float s = 0.f;
-#pragma unroll 1
-                for (int k = 0; k < K; ++k)
-                    s = fmaf(A[static_cast<size_t>(m) * K + k],
-                             WT ? W[static_cast<size_t>(k) * kSplitNO + n] : W[static_cast<size_t>(n) * K + k], s);
-                C[static_cast<size_t>(m) * kSplitNO + n] = s + bias_l[n];
+        // 16 tokens' results: lane r = token, acc[t] the channels c0 + 8 kg + 4 t on
+        auto put = [&](int sh, const f32x4 (&acc)[2]) {
+            if (16 * sh + r < rows) {
+                float* const out = C + static_cast<size_t>(lo + STEP * i + 16 * sh) * kSplitNO;  // uniform
+                const int at = unhoisted(r * kSplitNO + c0 + 8 * kg);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    *reinterpret_cast<f32x4*>(out + at + 4 * t) =
+                        acc[t] + *reinterpret_cast<const f32x4*>(bias_l + (at & (kSplitNO - 1)) + 4 * t);
             }
+        };
+        if (w_beyond || flagged(i & 1)) {  // the step on the float32 units, the operands from memory
+            const int rr = unhoisted(r), kk = unhoisted(kg * 4);
+            const int m = lo + STEP * i + rr, ch = c0 + 8 * (rr >> 2) + (rr & 3);  // tile t's row r: channel ch + 4 t
+            const float* const a[2] = {A + static_cast<size_t>(min(m, hi - 1)) * K + kk,
+                                       A + static_cast<size_t>(min(m + 16, hi - 1)) * K + kk};
+            f32x4 acc[2][2], x[2], w[2];
+#pragma unroll
+            for (int sh = 0; sh < 2; ++sh) acc[sh][0] = acc[sh][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            auto load = [&](int k) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    x[t] = *reinterpret_cast<const f32x4*>(a[t] + k);
+                    if constexpr (WT) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) w[t][e] = W[static_cast<size_t>(k + kk + e) * kSplitNO + ch + 4 * t];
+                    } else {
+                        w[t] = *reinterpret_cast<const f32x4*>(W + static_cast<size_t>(ch + 4 * t) * K + k + kk);
+                    }
+                }
+            };
+            load(0);
+#pragma unroll 1
+            for (int k = 16; k <= K; k += 16) {
+                const f32x4 xc[2] = {x[0], x[1]}, wc[2] = {w[0], w[1]};
+                load(min(k, K - 16));  // in flight during the MFMAs
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int sh = 0; sh < 2; ++sh)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+                            acc[sh][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[t][e], xc[sh][e], acc[sh][t], 0, 0, 0);
+            }
+            put(0, acc[0]);
+            put(1, acc[1]);
             wait_vm<0>();
             return;
         }
@@ -242,14 +281,7 @@ __global__ __launch_bounds__(kSplitWaves* kWave) __attribute__((amdgpu_waves_per
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (16 * sh + r < rows) {
-                float* const out = C + static_cast<size_t>(lo + STEP * i + 16 * sh) * kSplitNO;  // uniform
-                const int at = unhoisted(r * kSplitNO + c0 + 8 * kg);
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    *reinterpret_cast<f32x4*>(out + at + 4 * t) =
-                        acc[t] + *reinterpret_cast<const f32x4*>(bias_l + (at & (kSplitNO - 1)) + 4 * t);
-            }
+            put(sh, acc);
         }
     };
     // Step i + 1's rows were requested before step i - 1's stores (the wavefronts that split first) or step i's

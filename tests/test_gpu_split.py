@@ -101,3 +101,44 @@ def test_split_weight_gradient_beyond_the_split():
     over = ref[9, rest].abs() > 3.4e38
     assert torch.equal(gw[9, rest].isinf(), over) or ((gw[9, rest].isinf() == over) | (ref[9, rest].abs() > 3.39e38)).all()
     assert torch.allclose(gw[10:, rest].double(), ref[10:, rest], rtol=0, atol=2e-3)
+
+
+# operands whose third and second parts fall under bfloat16's smallest subnormal: every bit of them still counts
+@pytest.mark.parametrize('scale', [-100, -112, -120, -126])
+@pytest.mark.parametrize('K', [128, 256])
+def test_split_projection_of_small_values(scale, K):
+    M = 2304001 // K
+    x, w, _ = problem(M, K, 256)
+    small = torch.zeros(M, dtype=torch.bool)
+    small[[0, 70, M - 1]] = small[4000:4100] = True
+    x[0, small] = (1 + x[0, small].abs()) * 2.0 ** scale
+    w *= 2.0 ** 40
+    got = _native.value_proj(x.cuda(), w.cuda(), None).cpu().double()
+    ref = x.double() @ w.double().T
+    assert ((got - ref).abs() <= (K + 4) * EPS * (x.double().abs() @ w.double().abs().T)).all()
+    # small weights, and the input gradient, which reads them as stored
+    x, w, _ = problem(M, K, 256, seed=1)
+    x, w = x * 2.0 ** 40, (1 + w.abs()) * 2.0 ** scale
+    got = _native.value_proj(x.cuda(), w.cuda(), None).cpu().double()
+    ref = x.double() @ w.double().T
+    assert ((got - ref).abs() <= (K + 4) * EPS * (x.double().abs() @ w.double().abs().T)).all()
+    if K == 256:
+        gm, _, _ = _native.input_weight_grad(x.cuda(), w.cuda(), x.cuda())
+        ref = x.double() @ w.double()
+        assert ((gm.cpu().double() - ref).abs() <= (K + 4) * EPS * (x.double().abs() @ w.double().abs())).all()
+
+
+@pytest.mark.parametrize('scale', [-100, -112, -120, -126])
+def test_split_weight_gradient_of_small_values(scale):
+    M = 8193
+    gen = torch.Generator().manual_seed(2)
+    G, X = torch.randn(1, M, 256, generator=gen), torch.randn(1, M, 200, generator=gen) * 2.0 ** 40
+    G[0] = (1 + G[0].abs()) * 2.0 ** scale
+    gw, gb = _native.weight_grad(G.cuda(), X.cuda())
+    G64, X64 = G[0].double(), X[0].double()
+    assert ((gw.cpu().double() - G64.T @ X64).abs() <= 8 * EPS * (G64.abs().T @ X64.abs())).all()
+    G = torch.randn(1, M, 256, generator=gen) * 2.0 ** 40
+    X = (1 + torch.randn(1, M, 200, generator=gen).abs()) * 2.0 ** scale
+    gw, _ = _native.weight_grad(G.cuda(), X.cuda())
+    G64, X64 = G[0].double(), X[0].double()
+    assert ((gw.cpu().double() - G64.T @ X64).abs() <= 8 * EPS * (G64.abs().T @ X64.abs())).all()
