@@ -704,7 +704,11 @@ __global__ __launch_bounds__(256) void loc_attn_backward_kernel(LocAttnParams lp
 // (the counts are cleared during the sums for the next level).
 // D is a power of two from 4 to 64 (lane = channel tid % D), P > 0. The sums reach grad_value in another order than
 // the direct scatter's, so the two agree to float rounding.
+// TILE: self-attention at D = 4 (float32; scatter_tile_kernel takes 8 channels and more), in tiles of 8 x 4 pixels of a
+// level's map, which touch fewer pixels than 32 queries along one map row: backward of the DINO encoder's sampling, B2,
+// 512 us in consecutive queries, 412 in tiles; 5376 tokens B1 63.6 -> 52.3.
 constexpr int kBucketPix = 1024;  // bounding-box pixels per level at most
+constexpr int kBucketTileW = 3, kBucketTileH = 2;  // logs of 2: QT = 32 queries
 constexpr int kBucketEnt = 1024;  // corner entries per level at most: QT * P * 4 with QT * L * P <= 256
 
 // a bucketed corner: its coefficient a * w_c and the offset of its grad_out row in LDS (r * D)
@@ -783,15 +787,89 @@ __device__ __forceinline__ bool levels_hold_once(const Geom& g, LevelTokens t) {
     return !__any(shared);
 }
 
-template <typename T, int NTH>
+// Self-attention (Q = N) by tiles of 2^tw_shift x 2^th_shift pixels of the levels' maps, level by level: where the levels
+// tile the tokens, query q lies at token q's pixel. Every query is visited once wherever the levels lie: one whose token
+// several levels hold, in the first of them; those of no level, in tiles of a further map, as wide as a tile, of all the
+// tokens. Lane l holds level l's size and first token, read once (L <= 64); by whole wavefronts, every lane active.
+struct QueryTiles {
+    const Geom& g;
+    int w, h, lo, hi, tw_shift, th_shift, per_bh;
+    bool once;  // the levels hold each token once
+    __device__ __forceinline__ QueryTiles(const Geom& geom, int tw, int th) : g(geom), tw_shift(tw), th_shift(th) {
+        const int lane = lane_id(), ll = lane < g.L ? lane : 0;
+        w = static_cast<int>(g.shapes[2 * ll + 1]), h = static_cast<int>(g.shapes[2 * ll]);
+        const int64_t st = g.starts[ll];
+        lo = static_cast<int>(st), hi = static_cast<int>(st >> 32);
+        once = levels_hold_once(g, lane < g.L ? level_tokens(g, st, static_cast<int64_t>(w) * h) : LevelTokens{0, 0});
+        per_bh = once ? 0 : (g.N + (1 << (tw_shift + th_shift)) - 1) >> (tw_shift + th_shift);
+        for (int l = 0; l < g.L; ++l) {
+            int nbx;
+            per_bh += level_tiles(l, nbx);
+        }
+    }
+    __device__ __forceinline__ int width(int l) const { return __builtin_amdgcn_readlane(w, l); }
+    __device__ __forceinline__ int height(int l) const { return __builtin_amdgcn_readlane(h, l); }
+    __device__ __forceinline__ int64_t start(int l) const {
+        return static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(lo, l))) |
+               static_cast<int64_t>(__builtin_amdgcn_readlane(hi, l)) << 32;
+    }
+    __device__ __forceinline__ int level_tiles(int l, int& nbx) const {
+        nbx = (width(l) + (1 << tw_shift) - 1) >> tw_shift;
+        return nbx * ((height(l) + (1 << th_shift) - 1) >> th_shift);
+    }
+};
+
+// Tile `rest` of a (b, h), rows r: pixel (qx + r % 2^tw_shift, qy + r / 2^tw_shift) of level lq's map (L: the further one)
+struct QueryTile {
+    const QueryTiles& ts;
+    int lq = 0, wq, hq, qx, qy, nx, ny;
+    int64_t stq;
+    __device__ __forceinline__ QueryTile(const QueryTiles& tiles, int rest) : ts(tiles) {
+        int nbx = 1;
+        for (; lq < ts.g.L; ++lq) {
+            const int n = ts.level_tiles(lq, nbx);
+            if (rest < n) break;
+            rest -= n;
+        }
+        const bool further = lq == ts.g.L;
+        const int tw = 1 << ts.tw_shift, th = 1 << ts.th_shift;
+        wq = further ? tw : ts.width(lq), hq = further ? (ts.g.N + tw - 1) >> ts.tw_shift : ts.height(lq);
+        stq = further ? 0 : ts.start(lq);
+        if (further) nbx = 1;
+        qx = (rest % nbx) * tw, qy = (rest / nbx) * th;
+        nx = min(tw, wq - qx), ny = min(th, hq - qy);
+    }
+    // the token of row r; -1: none (past the map, or not in [0, N))
+    __device__ __forceinline__ int token(int r) const {
+        const int y = r >> ts.tw_shift, x = r & ((1 << ts.tw_shift) - 1);
+        const int64_t q = stq + static_cast<int64_t>(qy + y) * wq + qx + x;
+        return x < nx && y < ny && q >= 0 && q < ts.g.N ? static_cast<int>(q) : -1;
+    }
+    // its query; -1 also where another tile visits it
+    __device__ __forceinline__ int query(int r) const {
+        int q = token(r);
+        if (!ts.once)
+            for (int l = 0; l < lq; ++l)
+                if (q >= ts.start(l) && q < ts.start(l) + static_cast<int64_t>(ts.width(l)) * ts.height(l)) q = -1;
+        return q;
+    }
+    // whether no row has a query (uniform; each wavefront sees it for itself)
+    __device__ __forceinline__ bool empty() const {
+        if (ts.once) return false;
+        const int rows = 1 << (ts.tw_shift + ts.th_shift);
+        bool any = false;
+        for (int r0 = 0; r0 < rows; r0 += kWave) any |= query(min(r0 + lane_id(), rows - 1)) >= 0;
+        return !__any(any);
+    }
+};
+
+template <typename T, int NTH, bool TILE>
 __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void scatter_bucket_kernel(BucketParams bp) {
     using A = float;
     constexpr int NW = NTH / kWave;
     constexpr int LB = 8;  // levels whose bounding boxes are found together
     const Geom& g = bp.g;
     const int D = g.D, HD = g.H * g.D, LP = g.LP, P = g.P, QT = bp.QT;
-    const int tid = threadIdx.x, d = tid & (D - 1), grp = tid / D, ngrp = NTH / D;
-    const int wave = tid >> 6, lane = tid & (kWave - 1);
 
     __shared__ A gr[2 * NTH];                 // [QT][D] (QT * D <= 2 * NTH)
     __shared__ int etok[kBucketEnt];          // direct levels: corner token, -1 outside
@@ -805,11 +883,14 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void s
     __shared__ int wtot[NW];
 
     const T* __restrict__ go = static_cast<const T*>(bp.grad_out);
-    for (int i = tid; i < kBucketPix; i += NTH) cnt[i] = 0;
+    for (int i = threadIdx.x; i < kBucketPix; i += NTH) cnt[i] = 0;
 
     // One tile: rows r < QT of image b and head h, row r being query query_of(r) (-1: no query; its samples have
     // no corner in the map)
     auto tile = [&](int b, int h, auto query_of) {
+        int tid = threadIdx.x;
+        if constexpr (TILE) asm volatile("" : "+v"(tid));  // nothing that follows from it is kept from tile to tile
+        const int d = tid & (D - 1), grp = tid / D, ngrp = NTH / D, wave = tid >> 6, lane = tid & (kWave - 1);
         A* __restrict__ gv =
             static_cast<A*>(bp.grad_value) + static_cast<int64_t>(b) * g.N * HD + static_cast<int64_t>(h) * D;
         for (int i = tid; i < QT * D; i += NTH) {
@@ -992,11 +1073,25 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void s
         }
     };
 
-    const int unit = (blockIdx.x % kXcds) * bp.per_xcd + blockIdx.x / kXcds;
-    if (unit >= bp.units) return;  // the whole workgroup
-    const int qt = unit % bp.qtiles, bh = unit / bp.qtiles;
-    const int q0 = qt * QT, nq = g.Q - q0 < QT ? g.Q - q0 : QT;
-    tile(bh / g.H, bh % g.H, [&](int r) { return r < nq ? q0 + r : -1; });
+    if constexpr (!TILE) {
+        // QT consecutive queries
+        const int unit = (blockIdx.x % kXcds) * bp.per_xcd + blockIdx.x / kXcds;
+        if (unit >= bp.units) return;  // the whole workgroup
+        const int qt = unit % bp.qtiles, bh = unit / bp.qtiles;
+        const int q0 = qt * QT, nq = g.Q - q0 < QT ? g.Q - q0 : QT;
+        tile(bh / g.H, bh % g.H, [&](int r) { return r < nq ? q0 + r : -1; });
+    } else {
+        // the level sizes, and with them the count of the tiles, are on the device: a workgroup strides over them
+        const QueryTiles ts(g, kBucketTileW, kBucketTileH);
+        const int tiles = g.B * g.H * ts.per_bh;
+        for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+            const int bh = t / ts.per_bh;
+            const QueryTile qt(ts, t - bh * ts.per_bh);
+            if (qt.empty()) continue;
+            __syncthreads();  // every wavefront is done with the previous tile's LDS
+            tile(bh / g.H, bh % g.H, [&](int r) { return qt.query(r); });
+        }
+    }
 }
 
 // The same scatter for self-attention (Q = N; where the levels tile the tokens, query q lies at token q's pixel), a
@@ -1086,77 +1181,25 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
     if (tid < 2) s.alloc[tid] = s.ndirect[tid] = 0;
     if (tid < 16) s.touched[0][tid] = 0;
 
-    // lane l's: level l's size and first token, read once (a load would wait for the atomics before it); L <= 64
-    const int ll = lane < g.L ? lane : 0;
-    const int level_w = static_cast<int>(g.shapes[2 * ll + 1]), level_h = static_cast<int>(g.shapes[2 * ll]);
-    const int64_t level_st = g.starts[ll];
-    const int level_lo = static_cast<int>(level_st), level_hi = static_cast<int>(level_st >> 32);
-    auto width = [&](int l) { return __builtin_amdgcn_readlane(level_w, l); };
-    auto height = [&](int l) { return __builtin_amdgcn_readlane(level_h, l); };
-    auto start = [&](int l) {
-        return static_cast<int64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(level_lo, l))) |
-               static_cast<int64_t>(__builtin_amdgcn_readlane(level_hi, l)) << 32;
-    };
-    auto level_tiles = [&](int l, int& nbx) {
-        nbx = (width(l) + tp.tw - 1) >> tp.tw_shift;
-        return nbx * ((height(l) + tp.th - 1) >> tp.th_shift);
-    };
-    // Every query is visited once wherever the levels lie: one whose token several levels hold, in the first of them;
-    // those of no level, in tiles of a further map tw pixels wide of all the tokens
-    const bool once = levels_hold_once(
-        g, lane < g.L ? level_tokens(g, level_st, static_cast<int64_t>(level_w) * level_h) : LevelTokens{0, 0});
-    int per_bh = once ? 0 : (g.N + QT - 1) >> (tp.tw_shift + tp.th_shift);
-    for (int l = 0; l < g.L; ++l) {
-        int nbx;
-        per_bh += level_tiles(l, nbx);
-    }
-    const int tiles = g.B * g.H * per_bh;
+    const QueryTiles ts(g, tp.tw_shift, tp.th_shift);  // (read once: a load would wait for the atomics before it)
+    const int tiles = g.B * g.H * ts.per_bh;
     int par = 0;
     for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
-        const int bh = t / per_bh, b = bh / g.H, h = bh - b * g.H;
-        int rest = t - bh * per_bh, lq = 0, nbx = 1;
-        for (; lq < g.L; ++lq) {
-            const int n = level_tiles(lq, nbx);
-            if (rest < n) break;
-            rest -= n;
-        }
-        const bool further = lq == g.L;
-        const int wq = further ? tp.tw : width(lq), hq = further ? (g.N + tp.tw - 1) >> tp.tw_shift : height(lq);
-        const int64_t stq = further ? 0 : start(lq);
-        if (further) nbx = 1;
-        const int qx = (rest % nbx) * tp.tw, qy = (rest / nbx) * tp.th;
-        const int nx = min(tp.tw, wq - qx), ny = min(tp.th, hq - qy);
-        // the token of row r; -1: none (past the map, or not in [0, N))
-        auto token_of = [&](int r) {
-            const int y = r >> tp.tw_shift, x = r & (tp.tw - 1);
-            const int64_t q = stq + static_cast<int64_t>(qy + y) * wq + qx + x;
-            return x < nx && y < ny && q >= 0 && q < g.Q ? static_cast<int>(q) : -1;
-        };
-        // its query; -1 also where another tile visits it. By a whole wavefront: it reads the levels' lanes
-        auto query_of = [&](int r) {
-            int q = token_of(r);
-            if (!once)
-                for (int l = 0; l < lq; ++l)
-                    if (q >= start(l) && q < start(l) + static_cast<int64_t>(width(l)) * height(l)) q = -1;
-            return q;
-        };
-        if (!once) {  // a tile without a query, which every wavefront sees for itself
-            bool any = false;
-            for (int r0 = 0; r0 < QT; r0 += kWave) any |= query_of(min(r0 + lane, QT - 1)) >= 0;
-            if (!__any(any)) continue;
-        }
+        const int bh = t / ts.per_bh, b = bh / g.H, h = bh - b * g.H;
+        const QueryTile qt(ts, t - bh * ts.per_bh);
+        if (qt.empty()) continue;
         A* __restrict__ gv =
             static_cast<A*>(tp.grad_value) + static_cast<int64_t>(b) * g.N * HD + static_cast<int64_t>(h) * D;
 
         // lane l's: the window on level l, the tile's pixel centres there and a margin, inside the map
         int wx0, wy0, wbw, wbh;
         {
-            const int wl = level_w, hl = level_h;
-            const A sx = static_cast<A>(wl) / static_cast<A>(wq), sy = static_cast<A>(hl) / static_cast<A>(hq);
-            int xa = static_cast<int>(floorf((qx + 0.5f) * sx - 0.5f));
-            int xb = static_cast<int>(floorf((qx + nx - 0.5f) * sx - 0.5f)) + 1;
-            int ya = static_cast<int>(floorf((qy + 0.5f) * sy - 0.5f));
-            int yb = static_cast<int>(floorf((qy + ny - 0.5f) * sy - 0.5f)) + 1;
+            const int wl = ts.w, hl = ts.h;
+            const A sx = static_cast<A>(wl) / static_cast<A>(qt.wq), sy = static_cast<A>(hl) / static_cast<A>(qt.hq);
+            int xa = static_cast<int>(floorf((qt.qx + 0.5f) * sx - 0.5f));
+            int xb = static_cast<int>(floorf((qt.qx + qt.nx - 0.5f) * sx - 0.5f)) + 1;
+            int ya = static_cast<int>(floorf((qt.qy + 0.5f) * sy - 0.5f));
+            int yb = static_cast<int>(floorf((qt.qy + qt.ny - 0.5f) * sy - 0.5f)) + 1;
             const int cx = (xa + xb) / 2, cy = (ya + yb) / 2;
             if (xb - xa + 1 > kSide) xa = cx - (kSide - 1) / 2, xb = cx + (kSide - 1) / 2;  // around the centre
             if (yb - ya + 1 > kSide) ya = cy - (kSide - 1) / 2, yb = cy + (kSide - 1) / 2;
@@ -1171,7 +1214,7 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
 
         // this thread's samples: point jp of row r, level by level
         const int r = static_cast<int>(fast_div(tp.d_p, static_cast<uint32_t>(tid))), jp = tid - r * P;
-        const int qr = query_of(min(r, QT - 1)), q = r < QT ? qr : -1;
+        const int qr = qt.query(min(r, QT - 1)), q = r < QT ? qr : -1;
         const int64_t first = ((static_cast<int64_t>(b) * g.Q + (q >= 0 ? q : 0)) * g.H + h) * g.LP + jp;
         // the samples of kAhead levels, loaded and waited for before any of their atomics: a wavefront's vector memory
         // operations complete in order, and a wait inside the levels' loop would be one for the atomics
@@ -1196,15 +1239,15 @@ __global__ __launch_bounds__(NTH, 4) void scatter_tile_kernel(TileParams tp) {
         load(0);
         meet_lds();  // every wavefront is done with the previous tile's rows
         for (int i = tid; i < QT * D; i += kTileThreads) {
-            const int row = i >> tp.d_shift, qr = token_of(row);
+            const int row = i >> tp.d_shift, qr = qt.token(row);
             s.gr[i] = qr >= 0 ? go[(static_cast<int64_t>(b) * g.Q + qr) * HD + static_cast<int64_t>(h) * D + (i - row * D)]
                               : T(0);
         }
 
         loaded();
         for (int l = 0; l < g.L; ++l, par ^= 1) {
-            const int wl = width(l), hl = height(l);
-            const int64_t st = start(l);
+            const int wl = ts.width(l), hl = ts.height(l);
+            const int64_t st = ts.start(l);
             if (l > 0 && l % kAhead == 0) {
                 load(l);
                 loaded();
@@ -2421,7 +2464,18 @@ int scatter_bucket_go(const BackParams& p, hipStream_t stream) {
     bp.per_xcd = static_cast<int>((units + kXcds - 1) / kXcds);
     bp.d_lp = make_fastdiv(static_cast<uint32_t>(g.LP));
     bp.d_p = make_fastdiv(static_cast<uint32_t>(g.P));
-    hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH>), dim3(static_cast<unsigned>(bp.per_xcd * kXcds)),
+    if constexpr (sizeof(T) == 4) {  // (16-bit types come here from D = 8)
+        if (g.Q == g.N && g.D < 8 && bp.QT == 1 << (kBucketTileW + kBucketTileH) &&
+            static_cast<int64_t>(g.B) * g.H * g.N <= (int64_t{1} << 30)) {
+            // as many workgroups as the kernel's registers allow (three a CU), or as there may be tiles
+            const int64_t tiles = static_cast<int64_t>(g.B) * g.H * (bp.qtiles + 2 * g.L);
+            const int64_t grid = std::min<int64_t>(tiles, 3 * static_cast<int64_t>(cu_count()));
+            hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, true>), dim3(static_cast<unsigned>(grid)), dim3(NTH), 0,
+                               stream, bp);
+            return launched("sample backward scatter");
+        }
+    }
+    hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, false>), dim3(static_cast<unsigned>(bp.per_xcd * kXcds)),
                        dim3(NTH), 0, stream, bp);
     return launched("sample backward scatter");
 }

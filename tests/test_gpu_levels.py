@@ -16,6 +16,8 @@ def placed(kind, levels):
     size = [h * w for h, w in levels]
     starts = [sum(size[:l]) for l in range(len(size))]
     total = sum(size)
+    if kind == 'tiled':
+        return starts, total
     if kind == 'gaps':          # tokens before, between and after the levels that belong to none
         return [s + 3 + 5 * l for l, s in enumerate(starts)], total + 5 * len(size) + 4
     if kind == 'after':         # as a model with a few extra tokens at the end
@@ -86,3 +88,11 @@ def test_self_attention_gradients_large_tiles():
     # the 16-bit form from 131072 rows
     for kind in ('gaps', 'shared', 'same'):
         compare(kind, 4, None, 8, 32, [(55, 85), (28, 36), (14, 15)], 4, torch.bfloat16, 'encoder', masked=kind == 'gaps')
+
+
+@pytest.mark.parametrize('kind', (*KINDS, 'tiled'))
+def test_self_attention_gradients_of_narrow_heads(kind):
+    # four channels a head: 8 x 4-pixel tiles of the bucketed scatter; windows that fit and that do not
+    for where in ('encoder', 'uniform'):
+        compare(kind, 2, None, 3, 4, [(33, 49), (21, 35), (3, 5)], 4, torch.float32, where, masked=where == 'uniform')
+    compare(kind, 1, None, 2, 4, [(6, 9)], 8, torch.float32, 'encoder')
