@@ -704,9 +704,9 @@ __global__ __launch_bounds__(256) void loc_attn_backward_kernel(LocAttnParams lp
 // (the counts are cleared during the sums for the next level).
 // D is a power of two from 4 to 64 (lane = channel tid % D), P > 0. The sums reach grad_value in another order than
 // the direct scatter's, so the two agree to float rounding.
-// TILE: self-attention at D = 4 (float32; scatter_tile_kernel takes 8 channels and more), in tiles of 8 x 4 pixels of a
-// level's map, which touch fewer pixels than 32 queries along one map row: backward of the DINO encoder's sampling, B2,
-// 512 us in consecutive queries, 412 in tiles; 5376 tokens B1 63.6 -> 52.3.
+// TILE: self-attention that scatter_tile_kernel does not take or is not faster at, in tiles of 8 x 4 pixels of a level's
+// map, which touch fewer pixels than 32 queries along one map row (float32 D = 4, backward of the DINO encoder's
+// sampling, B2: 512 us in consecutive queries, 412 in tiles; 5376 tokens B1 63.6 -> 52.3).
 constexpr int kBucketPix = 1024;  // bounding-box pixels per level at most
 constexpr int kBucketTileW = 3, kBucketTileH = 2;  // logs of 2: QT = 32 queries
 constexpr int kBucketEnt = 1024;  // corner entries per level at most: QT * P * 4 with QT * L * P <= 256
@@ -2422,8 +2422,8 @@ int scatter_tile_shape_go(const BackParams& p, hipStream_t stream) {
     return launched("sample backward scatter");
 }
 
-// Below 32768 rows the consecutive-query form, whose tiles are done sooner, is the faster one (training step, it against
-// the query tiles: 1 x 8 x 3000 rows 81.1 us against 86.4 in float16, 94.0 / 99.8 in float32, 1 x 8 x 790 58.4 / 64.1; at
+// Below 32768 rows the bucketed form, whose tiles are done sooner, is the faster one (training step, it against the query
+// tiles: 1 x 8 x 3000 rows 81.1 us against 86.4 in float16, 94.0 / 99.8 in float32, 1 x 8 x 790 58.4 / 64.1; at
 // 1 x 8 x 5376, 43008 rows, 129 / 110)
 constexpr int64_t kTileMinRows = 32768;
 
@@ -2442,6 +2442,12 @@ int scatter_tile_go(const BackParams& p, hipStream_t stream) {
     if (rows < kTileMinRows) return 1;
     return scatter_tile_shape_go<T, 512>(p, stream);
 }
+
+// Rows from which the bucketed scatter of self-attention goes by 8 x 4-pixel tiles instead of consecutive queries, and
+// up to kTileMinRows (us of the sampling backward, consecutive queries against tiles, float16): D = 32 13680 rows 33.3 /
+// 38.6, 16000 34.6 / 32.4, 18000 38.0 / 33.5, 30912 62.1 / 49.0; D = 16 18000 26.2 / 27.3, 30912 42.2 / 35.7; D = 8 18000
+// 26.2 / 25.4, 30912 40.2 / 33.6. D = 4 at every size (see there).
+inline int64_t bucket_tile_min_rows(int D) { return D < 8 ? 0 : D < 32 ? 20000 : 16000; }
 
 template <typename T>
 int scatter_bucket_go(const BackParams& p, hipStream_t stream) {
@@ -2464,16 +2470,15 @@ int scatter_bucket_go(const BackParams& p, hipStream_t stream) {
     bp.per_xcd = static_cast<int>((units + kXcds - 1) / kXcds);
     bp.d_lp = make_fastdiv(static_cast<uint32_t>(g.LP));
     bp.d_p = make_fastdiv(static_cast<uint32_t>(g.P));
-    if constexpr (sizeof(T) == 4) {  // (16-bit types come here from D = 8)
-        if (g.Q == g.N && g.D < 8 && bp.QT == 1 << (kBucketTileW + kBucketTileH) &&
-            static_cast<int64_t>(g.B) * g.H * g.N <= (int64_t{1} << 30)) {
-            // as many workgroups as the kernel's registers allow (three a CU), or as there may be tiles
-            const int64_t tiles = static_cast<int64_t>(g.B) * g.H * (bp.qtiles + 2 * g.L);
-            const int64_t grid = std::min<int64_t>(tiles, 3 * static_cast<int64_t>(cu_count()));
-            hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, true>), dim3(static_cast<unsigned>(grid)), dim3(NTH), 0,
-                               stream, bp);
-            return launched("sample backward scatter");
-        }
+    const int64_t rows = static_cast<int64_t>(g.B) * g.H * g.N;
+    if (g.Q == g.N && bp.QT == 1 << (kBucketTileW + kBucketTileH) && rows >= bucket_tile_min_rows(g.D) &&
+        rows <= (int64_t{1} << 30)) {
+        // as many workgroups as the kernel's registers allow (three a CU), or as there may be tiles
+        const int64_t tiles = static_cast<int64_t>(g.B) * g.H * (bp.qtiles + 2 * g.L);
+        const int64_t grid = std::min<int64_t>(tiles, 3 * static_cast<int64_t>(cu_count()));
+        hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, true>), dim3(static_cast<unsigned>(grid)), dim3(NTH), 0, stream,
+                           bp);
+        return launched("sample backward scatter");
     }
     hipLaunchKernelGGL((scatter_bucket_kernel<T, NTH, false>), dim3(static_cast<unsigned>(bp.per_xcd * kXcds)),
                        dim3(NTH), 0, stream, bp);

@@ -79,9 +79,11 @@ def test_decoder_gradients(kind, dtype):
 @pytest.mark.parametrize('kind', KINDS)
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
 def test_self_attention_gradients(kind, dtype):
-    # as many queries as tokens, 32768 rows and more: a query counts once whether its token lies in no level, one or two
+    # as many queries as tokens: a query counts once whether its token lies in no level, one or two. 32768 rows and more,
+    # then under them
     compare(kind, 6, None, 4, 64, [(33, 49), (21, 35)], 4, dtype, 'encoder')
     compare(kind, 7, None, 5, 32, [(29, 40), (24, 31)], 4, dtype, 'encoder', masked=True)
+    compare(kind, 2, None, 8, 32, [(29, 40), (12, 16)], 4, dtype, 'encoder')
 
 
 def test_self_attention_gradients_large_tiles():

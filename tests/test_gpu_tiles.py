@@ -19,7 +19,9 @@ SHAPES = [
     (8, 3, 64, 4, [(31, 47), (16, 24)]),
     (6, 6, 16, 16, [(24, 39)]),
     (8, 8, 8, 2, [(25, 15), (40, 5)]),
-    (1, 2, 32, 4, [(31, 47), (16, 24)]),    # under 32768 rows: consecutive queries
+    (1, 2, 32, 4, [(31, 47), (16, 24)]),    # consecutive queries
+    (2, 8, 32, 4, [(31, 37), (16, 19)]),    # from 16000 rows (20000 under 32 channels) to 32768: 8 x 4 tiles
+    (2, 8, 8, 8, [(31, 37), (16, 19)]),
 ]
 
 
