@@ -2726,7 +2726,7 @@ int launch_transpose(int dtype, const void* src, void* dst, int64_t R, int64_t C
 
 // Whether the weight gradient of these operands runs on the split kernel: float32 with whole, aligned 16-byte rows.
 static bool wgrad_split_pays(int dtype, const void* G, const void* X, int64_t M, int64_t NO, int64_t K) {
-    return dtype == kF32 && split_size_pays(M, K) && NO % 4 == 0 && K % 4 == 0 &&
+    return dtype == kF32 && wgrad_split_size_pays(M, NO, K) && NO % 4 == 0 && K % 4 == 0 &&
            ((reinterpret_cast<uintptr_t>(G) | reinterpret_cast<uintptr_t>(X)) % 16) == 0;
 }
 

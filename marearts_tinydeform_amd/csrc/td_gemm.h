@@ -94,9 +94,17 @@ int launch_gemm_stream(int dtype, GemmParams p, hipStream_t stream, bool w_store
 // Sizes (rows x channels) from which float32 products are faster split: 6400 rows of 256 channels. Projection K = 256:
 // 5000 rows 13.4 us against 12.1 split, 8400 19.8 against 15.4, 2400 8.8 against 11.7 (the split kernel's start is 8
 // of them); both projection gradients, K = 256: 5000 rows 35.9 in the combined launch against 38.0, 8400 51.9 against
-// 47.5; 8400 x 384 84.7 against 73.1, 6000 x 512 106.6 against 82.0, 5000 x 128 21.9 against 27.5. One line for the
-// three products, so that each has the same bits whichever entry computes it.
+// 47.5; 8400 x 384 84.7 against 73.1, 6000 x 512 106.6 against 82.0, 5000 x 128 21.9 against 27.5. A product's line does
+// not ask which entry computes it, so that it has the same bits from each.
 inline bool split_size_pays(int64_t M, int64_t K) { return M >= 2048 && M * K >= 6400 * 256; }
+// The weight gradient G[M, NO]^T X[M, K] also needs two rows of tiles, or 20000 rows of 256 channels (both gradients, us,
+// one row of tiles: NO = 64, K = 256 6400 rows 25.3 against 26.5 split, 12800 38.2 / 39.1, 16800 42.8 / 43.5, 20000 57.9 /
+// 50.4; NO = 96, K = 512 8400 45.4 / 46.9, 10000 64.3 / 47.5; NO = 128, K = 1024 3200 39.2 / 40.7, 5000 64.3 / 49.4), or
+// the input gradient split beside it (NO = 128, K = 256 8400 36.5 / 38.8, 12800 43.3 / 38.3).
+inline bool wgrad_split_size_pays(int64_t M, int64_t NO, int64_t K) {
+    return split_size_pays(M, K) &&
+           (NO > 128 || M * K >= 20000 * 256 || (NO == 128 && K == 256 && split_size_pays(M, NO)));
+}
 bool gemm_split_fits(const GemmParams& p);
 bool gemm_split_pays(const GemmParams& p);
 int launch_gemm_split(GemmParams p, hipStream_t stream, bool w_stored = false);

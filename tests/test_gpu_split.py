@@ -76,9 +76,11 @@ def test_split_projection_of_unaligned_rows():
     assert (got - ref).abs().max() < 1e-4
 
 
-# tiles cut on both sides, one partial split, many; bias in the last, partial, tile of columns
+# tiles cut on both sides, one partial split, many; bias in the last, partial, tile of columns; up to 128 columns on
+# both sides of the line that those have for themselves
 @pytest.mark.parametrize('M,NO,K', [(6401, 256, 256), (20011, 256, 128), (4801, 384, 384), (9001, 100, 260),
-                                    (16003, 132, 200), (2048, 64, 1024)])
+                                    (16003, 132, 200), (2048, 64, 1024), (20003, 100, 260), (5003, 64, 1024),
+                                    (12800, 128, 256)])
 def test_split_weight_gradient(M, NO, K):
     gen = torch.Generator().manual_seed(1)
     G, X = torch.randn(1, M, NO, generator=gen), torch.randn(1, M, K, generator=gen)
