@@ -206,9 +206,10 @@ def train_times(cpu_args, steps, warmup):
 def gemm_kernel(M, K, NO, s):
     """Which value-projection kernel td_value_proj launches for an aligned [M, K] x [K, NO] problem (element size
     s), following its size rule: 16-bit with 256 outputs, K = 256 and at least 14000 rows (K = 128: 8000), or with
-    384 outputs, K = 384 and 10000 rows, takes the streaming kernel; 16-bit deep K (K >= 512, K % 64 == 0) on a grid of >= 200 tiles of 256 x 128, more than 256 of 128 x 128 or
-    from 8000 rows the direct-to-LDS kernels (persistent 256 x 256 tiles from 120 of them when NO % 16 == 0 and the
-    sizes stay below 2^31 elements, else 256 x 128 tiles);
+    384 outputs, K = 384 and more than 256 tiles of 128 x 128, takes the streaming kernel; 16-bit deep K (K >= 512,
+    K % 64 == 0) on a grid of >= 200 tiles of 256 x 128, more than 256 of 128 x 128 or from 8000 rows the direct-to-LDS
+    kernels (persistent 256 x 256 tiles from 120 of them when NO % 16 == 0 and the sizes stay below 2^31 elements, else
+    256 x 128 tiles);
     other 16-bit grids take register-operand tiles (32 x 32 to 64 x 64) up to 1100 tiles of 64 x 64 for K <= 256 and
     under 512 for deeper K, larger ones both operands through LDS;
     float32 takes register-operand tiles of 32 x 32 to 64 x 128."""
@@ -216,7 +217,7 @@ def gemm_kernel(M, K, NO, s):
     if s == 2:
         if NO == 256 and K in (128, 256) and M >= (14000 if K == 256 else 8000):
             return 'gemm_stream_kernel'
-        if NO == K == 384 and M >= 10000:
+        if NO == K == 384 and tiles_128 > 256:
             return 'gemm_stream_kernel'
         if K >= 512 and K % 64 == 0 and (-(-M // 256) * -(-NO // 128) >= 200 or tiles_128 > 256 or M >= 8000):
             lim = 1 << 31

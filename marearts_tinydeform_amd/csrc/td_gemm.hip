@@ -237,8 +237,9 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //   256 outputs: the streaming kernel (22) from 14000 rows at K = 256 (M = 16384 8.3 µs against 9.1 for 25, M = 16800
 //     9.1 against 11.2 for 13 and 12.2 for 25, M = 33600 12.2 against 15.4, M = 67200 17.6 against 23.5; it loses at
 //     12000 rows, 7.8 against 7.4 for 25, and at 8400, 7.5 against 7.1), from 8000 rows at K = 128 (M = 8400 5.4
-//     against 5.6 for 25, M = 16384 6.1 against 7.0); 384 outputs of K = 384: from 10000 rows (M = 12000 11.3 against
-//     13.3 for 13, M = 84253 40.7 against 51.3; at 8400 10.8 for both);
+//     against 5.6 for 25, M = 16384 6.1 against 7.0); 384 outputs of K = 384: from more than one round (256) of the
+//     128 x 128 tiles of 9 (M = 10880 11.2 against 10.7, M = 10881 11.2 against 19.0, M = 14000 11.8 against 19.2,
+//     M = 84253 40.7 against 51.3);
 //   deep K (K >= 512, K % 64 == 0) on a grid of at least 200 tiles of 256 x 128, or more than one round (256) of
 //     128 x 128 tiles, or from 8000 rows: the direct-to-LDS kernels, persistent 256 x 256 tiles (18) from 120 of
 //     them, else 256 x 128 (14) (C = 1024: M = 43520 87-89 µs for 18 against 97-100 for the same tiles one per
@@ -272,7 +273,7 @@ int pick_variant(int dtype, const GemmParams& p) {
         if (p.K <= 256) return tiles_64 <= 40 ? 24 : tiles_64 <= 100 ? 23 : tiles_64 <= 1100 ? 25 : tiles_128 < 1024 ? 5 : 2;
         return tiles_64 < 512 ? 25 : 2;
     }
-    if (gemm_stream_fits(dtype, p) && p.M >= (p.K == 256 ? 14000 : p.K == 384 ? 10000 : 8000)) return 22;
+    if (gemm_stream_fits(dtype, p) && (p.K == 384 ? tiles_128 > 256 : p.M >= (p.K == 256 ? 14000 : 8000))) return 22;
     const int64_t tiles_256x128 = ((p.M + 255) / 256) * static_cast<int64_t>((p.NO + 127) / 128);
     const int64_t tiles_256 = ((p.M + 255) / 256) * static_cast<int64_t>((p.NO + 255) / 256);
     if (p.K >= 512 && p.K % 64 == 0 && (tiles_256x128 >= 200 || tiles_128 > 256 || p.M >= 8000))

@@ -64,6 +64,15 @@ def test_streaming_kernel_needs_an_aligned_bias():
         assert _native.value_proj_plan(BF16, 67200, 256, 256, offsets={k: 8}) != 22
 
 
+def test_streaming_384_line():
+    # a product that one round of the 128 x 128 tiles holds stays there (10000 rows: 10.7 us against 11.1)
+    import bench
+    for dt in (F16, BF16):
+        for M, kern in ((8400, 9), (10000, 9), (10880, 9), (10881, 22), (20000, 22)):
+            assert _native.value_proj_plan(dt, M, 384, 384) == kern
+            assert bench.gemm_kernel(M, 384, 384, 2) == ('gemm_stream_kernel' if kern == 22 else 'gemm_lds_kernel')
+
+
 def test_persistent_tiles_need_their_alignments():
     # the persistent 256 x 256 tiles store 16 channels per lane as two 16-byte vectors and read the bias the same way
     assert _native.value_proj_plan(F16, 43520, 1024, 1024) == 18

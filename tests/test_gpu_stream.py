@@ -10,8 +10,8 @@ from test_gpu_parity import GEMM_EPS, assert_close, heads_of
 pytestmark = pytest.mark.gpu
 
 
-# shares of 39 or 40 tokens (a second step of 7 or 8), one past, whole steps, many steps off the step size
-@pytest.mark.parametrize('M', [10000, 10001, 16384, 36001, 70003])
+# shares of 42 or 43 tokens (a second step of 10 or 11), one past, whole steps, many steps off the step size
+@pytest.mark.parametrize('M', [10881, 11009, 16384, 36001, 70003])
 @pytest.mark.parametrize('bias', [True, False])
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 def test_streaming_384(M, bias, dtype):
