@@ -212,7 +212,8 @@ def gemm_kernel(M, K, NO, s):
     256 x 128 tiles);
     other 16-bit grids take register-operand tiles (32 x 32 to 64 x 64) up to 1100 tiles of 64 x 64 for K <= 256 and
     under 512 for deeper K, larger ones both operands through LDS;
-    float32 takes register-operand tiles of 32 x 32 to 64 x 128."""
+    float32 takes the split-operand kernel for 256 outputs of K = 256 from 6400 rows (K = 128: 12800), else
+    register-operand tiles of 32 x 32 to 64 x 128."""
     tiles_128 = -(-M // 128) * -(-NO // 128)
     if s == 2:
         if NO == 256 and K in (128, 256) and M >= (14000 if K == 256 else 8000):
@@ -229,6 +230,8 @@ def gemm_kernel(M, K, NO, s):
         if K <= 256:
             return 'gemm_mfma_kernel' if tiles_64 <= 1100 else 'gemm_lds_kernel'
         return 'gemm_mfma_kernel' if tiles_64 < 512 else 'gemm_lds_kernel'
+    if NO == 256 and K in (128, 256) and M * K >= 6400 * 256:
+        return 'gemm_split_kernel'
     return 'gemm_mfma_kernel'
 
 

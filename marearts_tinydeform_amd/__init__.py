@@ -118,8 +118,7 @@ def cost_features(B, Q, H, D, C, N, L, P, s, aligned=True):
     v = _native.value_proj_plan(pdt, M, K, NO, heads=H if hm else None, N=N if hm else None) if M * NO > 0 else -1
     mb, gf = M * (K + NO) * s / 1e6, 2.0 * M * K * NO / 1e9
     gemm = [1.0] + [0.0] * 10
-    split = s == 4 and v > 0 and NO == 256 and K in (128, 256) and M * K >= 6400 * 256 and not hm  # float32 on split operands
-    if v == 22 or split:
+    if v in (22, 26):
         gemm[1] = -(-(-(-M // CUS)) // 32) * 32 * (K + NO) * s * CUS / 1e6
         if s == 2 and K == 384:  # its steps move their bytes at 1 / 1.75 of the narrower ones' rate
             gemm[1] *= 1.75

@@ -2741,7 +2741,7 @@ int launch_input_weight_grad(int dtype, const void* G, const void* W, void* Wt, 
     // grad_memory = G . W with W read as stored
     const GemmParams sp{G, W, nullptr, gm, static_cast<int>(M), static_cast<int>(HD), static_cast<int>(C), 0, 0, 0};
     int rc = 0;
-    if (dtype == kF32 && gemm_split_pays(sp) && wgrad_split_pays(dtype, G, X, M, HD, C)) {
+    if (dtype == kF32 && gemm_split_pays(sp)) {
         rc = launch_gemm_split(sp, stream, true);
         if (rc != 0) return rc;
         return launch_wgrad(dtype, G, X, gw, gb, M, HD, C, workspace, ws_bytes, stream);

@@ -231,6 +231,7 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //   23 64 x 32   4 waves of 16 x 32, one chunk of 256/128, one stage
 //   24 32 x 32   2 waves of 16 x 32, one chunk of 256/128, one stage
 //   25 64 x 64   4 waves of 16 x 64, K chunks of 128/64, two stages
+//   26 the float32 streaming kernel on split operands (td_gemm_split.hip; gemm_split_pays)
 //   0  gemm_generic_kernel (float64, odd K, A or W not 16-byte aligned)
 //
 // Measured on MI355X (16-bit):
@@ -260,8 +261,8 @@ int go_mfma(GemmParams p, hipStream_t stream) {
 //   (K = NO = 256: M = 300 6.0 µs against 9.4 for 5), up to 100 64 x 32 (23) (M = 1200 6.8 against 9.5), up to 1100
 //   two-stage 64 x 64 (25) (M = 2400 9.2 against 9.7), then 64 x 64 one-chunk tiles (5) under 1024 tiles of 128 x 128
 //   (M = 33600 54.4 against 56.2), else A direct in 64 x 128 tiles (2); K >= 512: two-stage 64 x 64 (25) under 512
-//   tiles (M = 600, K = NO = 1024: 27.2 against 48.8 for 2), else 2. Of these, products that the split kernels compute
-//   faster on the bfloat16 units (gemm_split_pays) run there instead.
+//   tiles (M = 600, K = NO = 1024: 27.2 against 48.8 for 2), else 2. Before these, products that the split kernel
+//   computes faster on the bfloat16 units (26; gemm_split_pays says from which sizes).
 int pick_variant(int dtype, const GemmParams& p) {
     if (dtype != kF32 && dtype != kF16 && dtype != kBF16) return 0;
     const int E = dtype == kF32 ? 4 : 8;
@@ -270,6 +271,7 @@ int pick_variant(int dtype, const GemmParams& p) {
     const int64_t tiles_64 = ((p.M + 63) / 64) * static_cast<int64_t>((p.NO + 63) / 64);
     const int64_t tiles_128 = ((p.M + 127) / 128) * static_cast<int64_t>((p.NO + 127) / 128);
     if (dtype == kF32) {
+        if (gemm_split_pays(p)) return 26;
         if (p.K <= 256) return tiles_64 <= 40 ? 24 : tiles_64 <= 100 ? 23 : tiles_64 <= 1100 ? 25 : tiles_128 < 1024 ? 5 : 2;
         return tiles_64 < 512 ? 25 : 2;
     }
@@ -286,9 +288,6 @@ template <typename T>
 int launch_t(GemmParams p, hipStream_t stream, int variant) {
     constexpr int dt = std::is_same<T, float>::value ? kF32 : std::is_same<T, f16>::value ? kF16
                        : std::is_same<T, bf16>::value ? kBF16 : kF64;
-    if constexpr (dt == kF32) {
-        if (variant != 0 && gemm_split_pays(p)) return launch_gemm_split(p, stream);
-    }
     if constexpr (!std::is_same<T, double>::value) {
         switch (variant) {
             case 0: break;
@@ -305,6 +304,9 @@ int launch_t(GemmParams p, hipStream_t stream, int variant) {
                 break;
             case 14: case 18: return launch_gemm_dma(dt, p, stream, variant);
             case 22: return launch_gemm_stream(dt, p, stream);
+            case 26:
+                if constexpr (dt == kF32) return launch_gemm_split(p, stream);
+                break;
             default: break;
         }
         if (variant != 0) return set_error(-1, "value_proj: no tile variant %d for this dtype", variant);

@@ -5,7 +5,7 @@ kernel the rule can pick for any shape has at least one of these cases; the GPU 
 Kernel numbers (csrc/td_gemm.hip): 0 generic VALU; 2, 5, 23, 24, 25 A-in-registers MFMA tiles; 9, 13 both operands
 through LDS; 14 direct-to-LDS 256 x 128 tiles, one per workgroup; 18 persistent direct-to-LDS 256 x 256 tiles (one
 workgroup per CU walking its tiles; last tiles moved back to end at M and NO); 22 the streaming kernel (W resident in
-registers, tokens streamed through LDS).
+registers, tokens streamed through LDS); 26 the float32 streaming kernel on split operands.
 """
 
 import torch
@@ -14,8 +14,10 @@ F16, BF16, F32, F64 = torch.float16, torch.bfloat16, torch.float32, torch.float6
 
 # (B, N, C, HD) run in every dtype, every row checked: {dtype: kernel} for each shape
 SMALL = [
-    ((1, 8400, 256, 256), {F16: 25, BF16: 25, F32: 25, F64: 0}),
-    ((4, 9000, 256, 256), {F16: 22, BF16: 22, F32: 5, F64: 0}),
+    ((1, 8400, 256, 256), {F16: 25, BF16: 25, F32: 26, F64: 0}),
+    ((4, 9000, 256, 256), {F16: 22, BF16: 22, F32: 26, F64: 0}),
+    ((1, 20000, 256, 512), {F16: 13, BF16: 13, F32: 5, F64: 0}),
+    ((3, 1700, 256, 256), {F16: 25, BF16: 25, F32: 25, F64: 0}),
     ((2, 8192, 128, 1024), {F16: 13, BF16: 13, F32: 2, F64: 0}),
     ((2, 77, 40, 48), {F16: 24, BF16: 24, F32: 24, F64: 0}),
     ((1, 130, 96, 72), {F16: 24, BF16: 24, F32: 24, F64: 0}),

@@ -48,7 +48,7 @@ def test_every_reachable_kernel_has_a_parity_case():
         assert not missing, f'{dt}: kernels {sorted(missing)} are reachable but no GPU parity case runs them'
     # the sweep reaches every kernel of the rule (a guard against the sweep itself going stale)
     assert reach[F16] == reach[BF16] == {0, 9, 13, 14, 18, 22, 23, 24, 25}
-    assert reach[F32] == {0, 2, 5, 23, 24, 25}
+    assert reach[F32] == {0, 2, 5, 23, 24, 25, 26}
     assert reach[F64] == {0}
 
 
@@ -62,6 +62,17 @@ def test_streaming_kernel_needs_an_aligned_bias():
     # so must memory, weight and value
     for k in ('memory', 'weight', 'value'):
         assert _native.value_proj_plan(BF16, 67200, 256, 256, offsets={k: 8}) != 22
+
+
+def test_split_kernel_is_reported():
+    # the float32 kernel on split operands has a number of its own: row-major, aligned operands, from its line
+    assert _native.value_proj_plan(F32, 6400, 256, 256) == _native.value_proj_plan(F32, 12800, 128, 256) == 26
+    for M, K in ((6399, 256), (12799, 128)):
+        assert _native.value_proj_plan(F32, M, K, 256) != 26
+    for k in ('memory', 'weight', 'value'):
+        assert _native.value_proj_plan(F32, 67200, 256, 256, offsets={k: 8}) != 26
+    assert _native.value_proj_plan(F32, 67200, 256, 256, offsets={'bias': 4}) == 26     # read element by element
+    assert _native.value_proj_plan(F32, 67200, 256, 256, heads=8, N=67200) != 26
 
 
 def test_streaming_384_line():
@@ -98,9 +109,10 @@ def test_bench_names_the_kernel_the_rule_picks():
     import bench
     family = {0: 'gemm_generic_kernel', 2: 'gemm_mfma_kernel', 5: 'gemm_mfma_kernel', 23: 'gemm_mfma_kernel',
               24: 'gemm_mfma_kernel', 25: 'gemm_mfma_kernel', 9: 'gemm_lds_kernel', 13: 'gemm_lds_kernel',
-              14: 'gemm_dma_kernel', 18: 'gemm_dma_persistent_kernel', 22: 'gemm_stream_kernel'}
-    Ms = (300, 2400, 7999, 8000, 8400, 14000, 21760, 30001, 43520, 67200, 177784)
-    for dt, s in ((F16, 2), (BF16, 2)):
+              14: 'gemm_dma_kernel', 18: 'gemm_dma_persistent_kernel', 22: 'gemm_stream_kernel',
+              26: 'gemm_split_kernel'}
+    Ms = (300, 2400, 6399, 6400, 7999, 8000, 8400, 12799, 12800, 14000, 21760, 30001, 43520, 67200, 177784)
+    for dt, s in ((F16, 2), (BF16, 2), (F32, 4)):
         for M, K, NO in itertools.product(Ms, (128, 256, 512, 768, 1024), (256, 320, 512, 768, 1000, 1024)):
             got = bench.gemm_kernel(M, K, NO, s)
             want = family[_native.value_proj_plan(dt, M, K, NO)]
