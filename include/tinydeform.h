@@ -272,6 +272,14 @@ int td_sample_backward(int dtype, const void* value, const int64_t* spatial_shap
                        int64_t B, int64_t Q, int64_t N, int64_t H, int64_t D, int64_t L, int64_t P, void* stream);
 
 /*
+ * Whether td_sample_backward writes grad_value directly for these sizes, with grad_value_acc as scratch, where dtype (in
+ * float32 TD_ACC_SCRATCH too) and 16-byte aligned gradients allow it: 1 or 0, or a negative TD_E* code. A float32 caller
+ * needs a second buffer only where it is 1. value and grad_out are only inspected for their alignment.
+ */
+int td_sample_backward_plan(int dtype, const void* value, const void* grad_out, int64_t B, int64_t Q, int64_t N,
+                            int64_t H, int64_t D, int64_t L, int64_t P);
+
+/*
  * Projection, input side: grad_memory[M, C] = grad_value[M, HD] . value_weight[HD, C] on the library's GEMM.
  * weight_t: a workspace of HD*C elements of dtype, which receives value_weight^T.
  */

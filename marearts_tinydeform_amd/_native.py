@@ -37,6 +37,7 @@ SIGNATURES = {
     'td_layer_prologue': (_int, [_int, _vp, _vp, _vp, _i64, _i64] + [_vp] * 7 + [_i64] * 6 + [_vp]),
     'td_layer_fused_forward': (_int, [_int, _vp, _vp, _vp, _i64, _i64] + [_vp] * 13 + [_i64] * 9 + [_vp]),
     'td_layer_sample_forward': (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp] + [_i64] * 7 + [_vp]),
+    'td_sample_backward_plan': (_int, [_int, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64]),
     'td_sample_backward': (_int, [_int] + [_vp] * 11 + [_i64] * 7 + [_vp]),
     'td_input_grad': (_int, [_int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp]),
     'td_weight_grad_workspace': (_i64, [_int, _i64, _i64, _i64]),
@@ -462,9 +463,10 @@ def sample_backward(value, heads, spatial_shapes, level_start_index, sampling_lo
     lc, aw = sampling_locations.contiguous(), attention_weights.contiguous()
     sh, st = spatial_shapes.contiguous(), level_start_index.contiguous()
     acc = torch.empty((B, N, HD), dtype=acc_dtype(dt), device=dev)
-    # float32 (float64) sums are the gradient; from 2^18 corners on a float32 decoder's are binned in the accumulator's
-    # memory and written beside it
-    binned = dt == torch.float32 and B * Q * H * L * P * 4 >= 1 << 18 and Q * L * P * 4 < 16 * N
+    # float32 (float64) sums are the gradient, except where a float32 decoder's are binned in the accumulator's memory and
+    # written beside it
+    binned = dt == torch.float32 and lib_.td_sample_backward_plan(DTYPE_CODES[dt], v.data_ptr(), go.data_ptr(), B, Q, N,
+                                                                  H, HD // H, L, P) == 1
     gv = acc if acc.dtype == dt and not binned else torch.empty((B, N, HD), dtype=dt, device=dev)
     gl = torch.empty_like(lc)
     ga = torch.empty_like(aw)

@@ -535,6 +535,18 @@ extern "C" int td_value_proj_plan(int dtype, const void* memory, const void* wei
                            static_cast<int>(head_major_N > 0 ? H : 0));
 }
 
+extern "C" int td_sample_backward_plan(int dtype, const void* value, const void* grad_out, int64_t B, int64_t Q,
+                                       int64_t N, int64_t H, int64_t D, int64_t L, int64_t P) {
+    int64_t unused[8];
+    const int rc = check_plan_sizes(dtype, B, Q, N, H, D, L, P, unused);
+    if (rc != TD_OK) return rc;
+    if (B * Q * H * D == 0 || N == 0 || L * P == 0) return 0;
+    Geom g{nullptr, nullptr, static_cast<int>(B), static_cast<int>(Q), static_cast<int>(N), static_cast<int>(H),
+           static_cast<int>(D), static_cast<int>(L), static_cast<int>(P), nullptr};
+    set_levels(g, nullptr);
+    return sample_backward_binned(dtype, g, value, grad_out) ? 1 : 0;
+}
+
 extern "C" int td_sample_backward(int dtype, const void* value, const int64_t* spatial_shapes,
                                   const int64_t* level_start_index, const void* sampling_locations,
                                   const void* attention_weights, const uint8_t* padding_mask, const void* grad_out,

@@ -2530,22 +2530,23 @@ int loc_attn_backward_go(const BackParams& p, hipStream_t stream) {
 
 // The binned path (sort_count_kernel ... sort_reduce_kernel) at decoder densities, with the location and weight
 // gradients from loc_attn_backward_kernel; grad_value (the element type, aligned to four elements, not the
-// accumulator) is written directly. Returns 1 without launching when it does not apply: too few corners to pay for its five launches, a dense
-// problem (the bucketed scatter's), a head width other than 8..64 (a power of two), more than kSortMaxBins bins or
-// 2^25 rows, scratch that does not fit in the accumulator buffer (acc_bytes), or shapes loc_attn_backward_kernel
-// does not take (value or grad_out rows not 16-byte aligned).
+// accumulator) is written directly. sort_plan gives its parameters, or 1 where it does not apply: too few corners to
+// pay for its five launches, a dense problem (the bucketed scatter's), a head width other than 8..64 (a power of two),
+// more than kSortMaxBins bins or 2^25 rows, scratch that does not fit in the accumulator buffer, or shapes that
+// loc_attn_backward_kernel does not take (value or grad_out rows not 16-byte aligned).
 constexpr int64_t kSortMinCorners = int64_t{1} << 18;
 
 template <typename T>
-int sample_backward_sorted(const BackParams& p, void* grad_value_t, int64_t acc_bytes, hipStream_t stream) {
+int sort_plan(const BackParams& p, void* grad_value_t, SortParams& sp, LocAttnParams& lp) {
     const Geom& g = p.g;
-    if (grad_value_t == nullptr || grad_value_t == p.grad_value || reinterpret_cast<uintptr_t>(grad_value_t) % (4 * sizeof(T)) != 0 ||
+    if (grad_value_t == nullptr || grad_value_t == p.grad_value ||
+        reinterpret_cast<uintptr_t>(grad_value_t) % (4 * sizeof(T)) != 0 ||
         reinterpret_cast<uintptr_t>(p.grad_value) % 16 != 0 || !is_pow2(g.D) || g.D < 8 || g.D > 64 || g.LP <= 0 ||
         g.LP > 256 || g.L > kMaxLevelPoints || bucket_scatter_pays(g))
         return 1;
     const int64_t rows = static_cast<int64_t>(g.B) * g.Q * g.H;
     if (rows * g.LP * 4 < kSortMinCorners || rows >= (int64_t{1} << 25)) return 1;
-    SortParams sp{};
+    const int64_t acc_bytes = static_cast<int64_t>(g.B) * g.N * g.H * g.D * 4;
     sp.loc = p.loc;
     sp.attn = p.attn;
     sp.grad_out = p.grad_out;
@@ -2574,10 +2575,6 @@ int sample_backward_sorted(const BackParams& p, void* grad_value_t, int64_t acc_
     }
     sp.nb = static_cast<int>(nb);
     sp.maxch = static_cast<int>(maxch);
-    // the location and weight gradients' plan (1: its 16-byte loads do not fit these sizes); they run beside the scan
-    LocAttnParams lp;
-    const int rc = loc_attn_plan<T>(p, lp);
-    if (rc != 0) return rc;
     unsigned char* scratch = static_cast<unsigned char*>(p.grad_value);  // 16-byte aligned (checked above)
     sp.entries = reinterpret_cast<uint2*>(scratch);
     sp.items = reinterpret_cast<uint4*>(scratch + ent_bytes);
@@ -2585,6 +2582,18 @@ int sample_backward_sorted(const BackParams& p, void* grad_value_t, int64_t acc_
     sp.bin_start = sp.hist + BH * nb * sp.qtiles;
     sp.counters = sp.bin_start + BH * (nb + 1);
     sp.d_lp = make_fastdiv(static_cast<uint32_t>(g.LP));
+    // the location and weight gradients' plan (1: its 16-byte loads do not fit these sizes); they run beside the scan
+    return loc_attn_plan<T>(p, lp);
+}
+
+template <typename T>
+int sample_backward_sorted(const BackParams& p, void* grad_value_t, hipStream_t stream) {
+    const Geom& g = p.g;
+    SortParams sp{};
+    LocAttnParams lp;
+    const int rc = sort_plan<T>(p, grad_value_t, sp, lp);
+    if (rc != 0) return rc;
+    const int64_t BH = static_cast<int64_t>(g.B) * g.H, nb = sp.nb, maxch = sp.maxch;
     const unsigned tiles = static_cast<unsigned>(BH * sp.qtiles);
     const size_t lds = static_cast<size_t>(nb) * sizeof(int);
     hipLaunchKernelGGL(sort_count_kernel<T>, dim3(tiles), dim3(256), lds, stream, sp);
@@ -2649,10 +2658,9 @@ int launch_sample_backward(int dtype, const void* value, const Geom& g, const vo
     BackParams p{value, loc, attn, grad_out, grad_value, grad_loc, grad_attn, g, 1};
     *direct = false;
     if (dtype != kF64 && (reinterpret_cast<uintptr_t>(grad_value) % 8) == 0) {
-        const int rs = dtype == kF32   ? sample_backward_sorted<float>(p, acc_scratch ? grad_value_t : nullptr, acc_bytes,
-                                                                        stream)
-                       : dtype == kF16 ? sample_backward_sorted<f16>(p, grad_value_t, acc_bytes, stream)
-                                       : sample_backward_sorted<bf16>(p, grad_value_t, acc_bytes, stream);
+        const int rs = dtype == kF32   ? sample_backward_sorted<float>(p, acc_scratch ? grad_value_t : nullptr, stream)
+                       : dtype == kF16 ? sample_backward_sorted<f16>(p, grad_value_t, stream)
+                                       : sample_backward_sorted<bf16>(p, grad_value_t, stream);
         if (rs != 1) {
             *direct = rs == 0;
             return rs;
@@ -2670,6 +2678,21 @@ int launch_sample_backward(int dtype, const void* value, const Geom& g, const vo
         case kBF16: return sample_backward_t<bf16>(p, stream);
         case kF64: return sample_backward_t<double>(p, stream);
         default: return set_error(-2, "unknown dtype code %d", dtype);
+    }
+}
+
+bool sample_backward_binned(int dtype, const Geom& g, const void* value, const void* grad_out) {
+    // any buffers of the right alignment, which the plan's pointers are counted from and nothing reads
+    void* const acc = reinterpret_cast<void*>(uintptr_t{1} << 12);
+    void* const gvt = reinterpret_cast<void*>(uintptr_t{1} << 13);
+    const BackParams p{value, acc, acc, grad_out, acc, acc, acc, g, 1};
+    SortParams sp{};
+    LocAttnParams lp;
+    switch (dtype) {
+        case kF32: return sort_plan<float>(p, gvt, sp, lp) == 0;
+        case kF16: return sort_plan<f16>(p, gvt, sp, lp) == 0;
+        case kBF16: return sort_plan<bf16>(p, gvt, sp, lp) == 0;
+        default: return false;
     }
 }
 

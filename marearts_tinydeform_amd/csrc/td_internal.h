@@ -125,6 +125,9 @@ int project_forward(int dtype, const void* memory, const void* value_weight, con
 int launch_sample_backward(int dtype, const void* value, const Geom& g, const void* loc, const void* attn,
                            const void* grad_out, void* grad_value, void* grad_value_t, void* grad_loc, void* grad_attn,
                            hipStream_t stream, bool* direct, bool acc_scratch);
+// Whether it bins the corners by token (grad_value_t written directly, the accumulator scratch) for these sizes and
+// 16-byte aligned gradients; value and grad_out are looked at for their alignment only
+bool sample_backward_binned(int dtype, const Geom& g, const void* value, const void* grad_out);
 // dst[i] = src[i] rounded from the accumulation type to dtype
 int launch_convert(int dtype, const void* src_acc, void* dst, int64_t n, hipStream_t stream);
 // dst [Cc, R] = src [R, Cc]^T

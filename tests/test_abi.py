@@ -37,7 +37,7 @@ def test_header_declares_the_entry_points():
                                   'td_layer_fused_forward', 'td_layer_prologue', 'td_layer_sample_forward',
                                   'td_probe_atomic', 'td_probe_empty', 'td_probe_gather',
                                   'td_project_forward', 'td_project_forward_noalloc', 'td_sample_backward',
-                                  'td_sample_forward',
+                                  'td_sample_backward_plan', 'td_sample_forward',
                                   'td_sample_forward_heads', 'td_sample_forward_masked', 'td_sample_forward_v2',
                                   'td_sample_plan',
                                   'td_value_proj', 'td_value_proj_heads', 'td_value_proj_plan', 'td_version',
@@ -253,3 +253,18 @@ def test_weight_grad_workspace_plan(lib, dtype, M, NO, K):
     s = max(splits(1), splits(2 if dtype != 3 and K >= 512 else 1))
     elem = 8 if dtype == 3 else 4
     assert lib.td_weight_grad_workspace(dtype, M, NO, K) == s * (NO * K + NO) * elem
+
+
+def test_sample_backward_plan_says_what_a_caller_has_to_allocate(lib):
+    # B, Q, N, H, D, L, P -> whether a float32 decoder's value gradient is binned (and needs a buffer beside the sums)
+    aligned = 4096
+    for sizes, want in (((8, 300, 8400, 8, 32, 3, 4), 1), ((8, 300, 8400, 8, 8, 3, 4), 1),
+                        ((8, 300, 8400, 8, 4, 3, 4), 0),         # head widths it does not take
+                        ((8, 300, 8400, 8, 24, 3, 4), 0), ((8, 300, 8400, 8, 128, 3, 4), 0),
+                        ((2, 350, 3150, 8, 8, 3, 4), 0),         # its entries do not fit in the sums' memory
+                        ((1, 300, 8400, 8, 32, 3, 4), 0),        # under 2^18 corners
+                        ((2, 8400, 8400, 8, 32, 3, 4), 0),       # as many queries as tokens
+                        ((1, 0, 8400, 8, 32, 3, 4), 0)):
+        assert lib.td_sample_backward_plan(0, aligned, aligned, *sizes) == want, sizes
+    assert lib.td_sample_backward_plan(0, aligned, aligned + 4, 8, 300, 8400, 8, 32, 3, 4) == 0
+    assert lib.td_sample_backward_plan(0, aligned, aligned, -1, 300, 8400, 8, 32, 3, 4) < 0

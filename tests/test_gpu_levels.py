@@ -74,6 +74,7 @@ def test_decoder_gradients(kind, dtype):
     # 2^18 corners and more: the binned value gradient. A hot spot makes split bins
     compare(kind, 2, 350, 8, 32, [(40, 60), (20, 30), (10, 15)], 4, dtype, 'uniform')
     compare(kind, 2, 350, 8, 16, [(40, 60), (20, 30), (10, 15)], 4, dtype, 'clustered', masked=True)
+    compare(kind, 3, 300, 8, 8, [(60, 80), (30, 40), (15, 20)], 4, dtype, 'clustered')
 
 
 @pytest.mark.parametrize('kind', KINDS)

@@ -100,3 +100,18 @@ def test_binned_float32_value_gradient(D, masked):
                                         torch.cuda.current_stream().cuda_stream)
     assert rc == 0 and torch.equal(acc, out)
     assert torch.allclose(gv, acc, rtol=1e-4, atol=1e-4) and torch.allclose(ga, ga2, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize('D,binned', [(32, True), (24, False), (128, False)])
+def test_float32_decoders_second_buffer(D, binned):
+    # a float32 value gradient takes a second buffer of its size only where its sums are binned
+    levels, B, Q, H, P = [(40, 60), (20, 30), (10, 15)], 2, 350, 8, 4
+    N = sum(h * w for h, w in levels)
+    args = [t.cuda() for t in workload(B, Q, H, D, 8, levels, P, torch.float32)[3:7]]
+    value, go = torch.randn(B, N, H * D, device='cuda'), torch.randn(B, Q, H * D, device='cuda')
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    grads = _native.sample_backward(value, H, *args, go)
+    size = value.numel() * 4
+    extra = torch.cuda.max_memory_allocated() - before - sum(t.numel() * 4 for t in grads)
+    assert (extra >= size) if binned else extra < size // 2
