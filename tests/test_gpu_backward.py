@@ -237,9 +237,9 @@ def test_decoder_sorted_value_gradients(dtype, D, shape, Q, with_mask):
 @pytest.mark.parametrize('dtype,D', [(torch.float16, 32), (torch.bfloat16, 16), (torch.float32, 8)])
 @pytest.mark.parametrize('with_mask', [False, True])
 def test_self_attention_tile_gradients(dtype, D, with_mask):
-    # as many queries as tokens: the bucketed scatter takes 8 x 4-pixel tiles of each level's map (query q at token
-    # q), here on maps whose sides are not multiples of 8 or 4 (tiles cut at the right and bottom edges) and a map
-    # narrower than a tile; encoder locations and uniform ones (every window then too large: the direct path)
+    # as many queries as tokens, of few rows (5028): the bucketed scatter by consecutive queries, on maps whose rows are
+    # not multiples of 32 and a map of fewer pixels; encoder locations and uniform ones (every window then too large: the
+    # direct path). More rows, and with them the query tiles: test_gpu_tiles.py; D = 4: test_gpu_levels.py
     levels = [(25, 37), (13, 19), (7, 10), (3, 5)]
     N = sum(h * w for h, w in levels)
     mask = (torch.rand(1, N, generator=torch.Generator().manual_seed(4)) < 0.2) if with_mask else None

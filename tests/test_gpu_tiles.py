@@ -45,6 +45,25 @@ def test_tile_scatter(shape, dtype):
         check(f'tiles {shape} {dtype} d{n}', grads[n], ref[n], dtype)
 
 
+# 16 x 16, 16 x 8 and 8 x 4 tiles and consecutive queries: in float32 (which has no 16 x 16), with padded tokens in and
+# outside the windows, and with locations all over the map, whose corners are mostly added directly
+@pytest.mark.parametrize('shape', [SHAPES[0], SHAPES[2], SHAPES[4], SHAPES[7], SHAPES[6]])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+@pytest.mark.parametrize('masked', [False, True])
+def test_tile_scatter_masked_and_far(shape, dtype, masked):
+    B, H, D, P, levels = shape
+    N = sum(h * w for h, w in levels)
+    mask = torch.rand(B, N, generator=torch.Generator().manual_seed(3)) < 0.25 if masked else None
+    for where in ('encoder', 'uniform'):
+        args = workload(B, N, H, D, 64, levels, P, dtype, loc_dist=where, seed=7)
+        args[5] = (args[5].float() * 1024).round().div(1024).to(dtype)     # pixels that do not hang on rounding
+        go = grad_out_for(args)
+        grads, _ = gpu_grads(args, go, dtype, mask=mask)
+        ref = gridsample.deform_attn_grads(*args, go.to(dtype), padding_mask=mask)
+        for n in NAMES:
+            check(f'tiles {shape} {dtype} {where} masked={masked} d{n}', grads[n], ref[n], dtype)
+
+
 def test_tile_scatter_keeps_infinities_where_they_belong():
     # an infinite grad_out row reaches the pixels it samples and no other, in float16 too
     levels = [(80, 100), (40, 50)]
