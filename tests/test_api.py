@@ -126,6 +126,18 @@ def test_cost_features_follow_the_launch_plans():
     assert fg[1] == pytest.approx(9 * 32 * 512 * 2 * 256 / 1e6)
 
 
+def test_auto_crossover_of_the_split_float32_projection():
+    # the float32 kernel on split operands has its start priced: measured (us, fused / project), C = 256: B1 Q900 24.3 /
+    # 28.0, B4 Q300 30 / 45, B8 Q300 47 / 62, B4 Q900 70 / 47, B8 Q900 128 / 84
+    _, fg, _ = td.cost_features(1, 900, 8, 32, 256, 8400, 3, 4, 4)
+    assert fg[11] == 1.0 and fg[7] == fg[8] == fg[10] == 0.0 and fg[1] == pytest.approx(64 * 512 * 4 * 256 / 1e6)
+    _, fg, _ = td.cost_features(1, 900, 8, 32, 256, 5000, 3, 4, 4)    # under its line: the tiles
+    assert fg[11] == 0.0 and fg[7] > 0
+    for B, Q, want in ((1, 900, 'fused'), (4, 300, 'fused'), (8, 300, 'fused'), (4, 900, 'project'), (8, 900, 'project')):
+        memory = torch.empty(B, 8400, 256)
+        assert td.choose_mode(memory, torch.empty(256, 256), torch.empty(B, Q, 8, 3, 4, 2)) == want
+
+
 def test_auto_crossover_moves_with_queries_batch_and_channels():
     # RT-DETR 640, 16-bit (measured on MI355X): fused at batch 1 up to 900 queries (14.1 against 14.6 µs at 900),
     # project from 600 queries at batch 4; C=1024 / 16 heads / 64 samples (the limit shape) switches to project by
