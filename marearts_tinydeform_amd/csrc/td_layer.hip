@@ -176,15 +176,16 @@ bool prologue_wants_gemm(int dtype, const Geom& g, int64_t Cq) {
 int launch_prologue(int dtype, const LayerArgs& layer, const Geom& g, hipStream_t stream, int route) {
     if (layer.loc_out == nullptr || layer.attn_out == nullptr)
         return set_error(-1, "layer prologue: locations and weights need output buffers");
-    // route 0: by the projections' multiply-adds. In 16 bits, where both projections share a launch (gemm_pair_kernel)
-    // and mostly the finalize too, the GEMM route from 1.2e8 (us, single kernel against GEMM route): fp16 C = 256, 8
-    // heads x 16 samples: 900 queries (0.9e8) 7.6 against 7.9, 1800 10.2 / 8.2, 3600 15.9 / 8.8, 7200 24.8 / 13.3; 8
-    // heads x 12 samples: 2100 10.2 / 9.3, 7200 22.0 / 18.2; C = 512 300 queries (1.2e8) 10.0 / 9.3, 1200 19.1 / 9.7;
-    // C = 1024 300 queries 15.5 / 12.0. With two launches and a finalize of its own (other types and sizes) from 8e8
-    // (600 queries, 16 heads x 64 samples, 1.9e9: 45 against 72).
+    // route 0: by the projections' multiply-adds (us, single kernel against GEMM route). In 16 bits both projections share
+    // a launch (gemm_pair_kernel). Where it finalizes too (a power of two of samples), from 1.2e8: fp16 C = 256, 8 heads x
+    // 16 samples 900 queries (0.9e8) 7.6 / 7.9, 1800 10.5 / 8.9, 3600 15.6 / 9.1, 7200 24.6 / 13.2; C = 512 900 queries
+    // 10.4 / 9.9; C = 1024, 16 heads x 64, 50 queries 30.2 / 12.6. With a finalize of its own from 2e8: 8 heads x 12
+    // samples 1800 queries (1.3e8) 9.9 / 10.6, 2400 10.8 / 10.9, 3600 14.2 / 11.6, 7200 22.5 / 18.3. With two launches and
+    // a finalize (other types and sizes) from 8e8 (600 queries, 16 heads x 64 samples, 1.9e9: 72 / 45).
     const double macs = static_cast<double>(g.B) * g.Q * g.H * 3 * g.LP * layer.Cq;
     const bool large = prologue_wants_gemm(dtype, g, layer.Cq);
-    const bool pair = (dtype == kF16 || dtype == kBF16) && macs >= 1.2e8;
+    const bool finalizes = g.LP >= 4 && (g.LP & (g.LP - 1)) == 0;
+    const bool pair = (dtype == kF16 || dtype == kBF16) && macs >= (finalizes ? 1.2e8 : 2e8);
     if (dtype != kF64 && (route == 2 || (route == 0 && (large || pair)))) {
         const bool pair_only = route == 0 && !large;
         int rc = 1;

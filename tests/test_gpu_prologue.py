@@ -10,11 +10,12 @@ from marearts_tinydeform_amd.reference import layer_locations_reference
 pytestmark = pytest.mark.gpu
 
 
-# below 1.2e8 multiply-adds (one kernel); above, finalized by the projections (16 samples) and apart (12), ragged
-# rows, no position embeddings; above with channels the two projections' launch does not take
+# below 1.2e8 multiply-adds (one kernel); above, finalized by the projections (16 samples), ragged rows, no position
+# embeddings; with 12 samples, finalized apart, on both sides of 2e8; above with channels the two projections' launch does
+# not take
 @pytest.mark.parametrize('B,Q,C,H,L,P,pos', [(1, 900, 256, 8, 4, 4, True), (3, 417, 256, 8, 4, 4, True),
-                                             (3, 567, 256, 8, 3, 4, True), (2, 331, 384, 12, 4, 4, False),
-                                             (3, 500, 264, 8, 4, 4, True)])
+                                             (3, 567, 256, 8, 3, 4, True), (3, 967, 256, 8, 3, 4, True),
+                                             (2, 331, 384, 12, 4, 4, False), (3, 500, 264, 8, 4, 4, True)])
 @pytest.mark.parametrize('dtype', [torch.float16, torch.bfloat16])
 def test_prologue_matches_float64(B, Q, C, H, L, P, pos, dtype):
     levels = [(40 >> l, 56 >> l) for l in range(L)]
