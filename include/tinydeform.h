@@ -264,6 +264,7 @@ int td_sample_plan(int dtype, int64_t B, int64_t Q, int64_t N, int64_t H, int64_
  *                               TD_ACC_SCRATCH lets float32 do the same (grad_value then given, and not
  *                               grad_value_acc itself);
  *   grad_loc [B, Q, H, L, P, 2], grad_attn [B, Q, H, L, P]: dtype.
+ * The levels may lie anywhere: a token of no level has a value gradient of 0, one that levels share the sum of theirs.
  * padding_mask as in td_sample_forward_masked. Limits as td_sample_forward, and D <= 256.
  */
 int td_sample_backward(int dtype, const void* value, const int64_t* spatial_shapes, const int64_t* level_start_index,

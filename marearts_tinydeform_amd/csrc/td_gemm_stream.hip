@@ -314,7 +314,9 @@ int stream_t(GemmParams p, hipStream_t stream) {
 
 }  // namespace
 
-// The bias is read with 16-byte loads, so it must be 16-byte aligned like the other operands.
+// The bias is read with 16-byte loads, so it must be 16-byte aligned like the other operands. The widths are those whose W
+// a workgroup's registers hold (a square one up to 384) in whole pairs of 16-channel tiles a wavefront (outputs a
+// multiple of 128); wider outputs of a narrow K (384 or 512 of 256) would fit and were not measured.
 bool gemm_stream_fits(int dtype, const GemmParams& p) {
     const uintptr_t al = reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.w) |
                          reinterpret_cast<uintptr_t>(p.c) | reinterpret_cast<uintptr_t>(p.bias);
