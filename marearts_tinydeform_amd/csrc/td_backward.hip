@@ -787,10 +787,11 @@ __device__ __forceinline__ bool levels_hold_once(const Geom& g, LevelTokens t) {
     return !__any(shared);
 }
 
-// Self-attention (Q = N) by tiles of 2^tw_shift x 2^th_shift pixels of the levels' maps, level by level: where the levels
-// tile the tokens, query q lies at token q's pixel. Every query is visited once wherever the levels lie: one whose token
-// several levels hold, in the first of them; those of no level, in tiles of a further map, as wide as a tile, of all the
-// tokens. Lane l holds level l's size and first token, read once (L <= 64); by whole wavefronts, every lane active.
+// Self-attention (Q = N) by tiles of 2^tw_shift x 2^th_shift pixels of the levels' maps, level by level: where the
+// levels tile the tokens, query q lies at token q's pixel. Every query is visited once wherever the levels lie: one
+// whose token several levels hold, in the first of them; those of no level, in tiles of a further map, as wide as a
+// tile, of all the tokens. Lane l holds level l's size and first token, read once (L <= 64): made by whole wavefronts,
+// and asked by ones whose first L lanes at least are active.
 struct QueryTiles {
     const Geom& g;
     int w, h, lo, hi, tw_shift, th_shift, per_bh;
@@ -819,7 +820,8 @@ struct QueryTiles {
     }
 };
 
-// Tile `rest` of a (b, h), rows r: pixel (qx + r % 2^tw_shift, qy + r / 2^tw_shift) of level lq's map (L: the further one)
+// Tile `rest` of a (b, h), rows r: pixel (qx + r % 2^tw_shift, qy + r / 2^tw_shift) of level lq's map (L: the further
+// one)
 struct QueryTile {
     const QueryTiles& ts;
     int lq = 0, wq, hq, qx, qy, nx, ny;
@@ -1094,10 +1096,10 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(6))) void s
     }
 }
 
-// The same scatter for self-attention (Q = N; where the levels tile the tokens, query q lies at token q's pixel), a
-// workgroup a tile of 16 x 16 or 16 x 8 pixels of a level's map: those queries of one head touch 10.2 and 7.9 times fewer pixels than they have corners on
-// DINO-style inputs (8 x 4 pixels: 4.3), and the float atomics, one D-wide line a touched pixel, run at 320 G lanes/s
-// whatever else is done (200 and 260 us at the DINO encoder). So the rest has to run beside them: the barriers wait for
+// The same scatter for self-attention (QueryTiles), a workgroup a tile of 16 x 16 or 16 x 8 pixels of a level's map:
+// those queries of one head touch 10.2 and 7.9 times fewer pixels than they have corners on DINO-style inputs (8 x 4
+// pixels: 4.3), and the float atomics, one D-wide line a touched pixel, run at 320 G lanes/s whatever else is done (200
+// and 260 us at the DINO encoder). So the rest has to run beside them: the barriers wait for
 // LDS only, nothing inside a tile waits for a load, and a level costs three barriers:
 //   * a thread a sample: its corners inside the level's window rank themselves within their pixel (an integer LDS
 //     atomic each); a corner outside it is listed for an atomic of its own. The window is the tile's image on the
